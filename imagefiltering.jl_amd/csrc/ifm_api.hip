@@ -1133,18 +1133,22 @@ int ifm_imfilter_iir(ifm_ctx *ctx, const ifm_array *in, ifm_array *out, const if
       if (vi.d.data != vo.d.data || vi.d.dtype != vo.d.dtype)
         HIPCHK(launch_fir1d(vi.d, zero, vo.d, zero, vi.d.n, p, b->style, (float)b->fill, st));
     } else {
-      Dense4 src = vi.d;
+      // Every stage but the first runs in place on one FP64 buffer: the output
+      // itself if it is F64.  The last stage writes the output's eltype where
+      // its lines are held in registers.
+      const auto axis_n = [&](size_t s) { return vi.d.n[g.inv[factors[live[s]].axis]]; };
+      const bool direct = iir_in_registers(axis_n(live.size() - 1));
+      Dense4 buf = vi.d;
+      buf.dtype = IFM_F64;
+      if (vo.d.dtype == IFM_F64) {
+        buf.data = vo.d.data;
+      } else if (live.size() > 1 || !direct) {
+        buf.data = slot_buffer(ctx, S_TMP1, (size_t)cnt * sizeof(double));
+        if (!buf.data) return fail(ctx, IFM_E_NOMEM, "device allocation failed (temporary)");
+      }
       for (size_t s = 0; s < live.size(); ++s) {
         const ifm_iir &k = factors[live[s]];
-        const bool last = s + 1 == live.size();
-        Dense4 dst = vi.d;
-        dst.dtype = IFM_F64;
-        if (last && vo.d.dtype == IFM_F64) {
-          dst.data = vo.d.data;
-        } else {
-          dst.data = slot_buffer(ctx, (s & 1) ? S_TMP2 : S_TMP1, (size_t)cnt * sizeof(double));
-          if (!dst.data) return fail(ctx, IFM_E_NOMEM, "device allocation failed (temporary)");
-        }
+        Dense4 src = s == 0 ? vi.d : buf, dst = s + 1 == live.size() && direct ? vo.d : buf;
         IirCoef c;
         for (int i = 0; i < 3; ++i) {
           c.a[i] = k.a[i];
@@ -1153,16 +1157,15 @@ int ifm_imfilter_iir(ifm_ctx *ctx, const ifm_array *in, ifm_array *out, const if
         c.scale = k.scale;
         for (int i = 0; i < 9; ++i) c.M[i] = k.M[i];
         HIPCHK(launch_iir(src, dst, g.inv[k.axis], c, isfill, b->fill, st));
-        src = dst;
       }
-      if (src.data != vo.d.data) {
+      if (!direct && buf.data != vo.d.data) {
         FirPass p;
         p.axis = 0;
         p.len = 1;
         p.first = 0;
         p.taps[0] = 1.f;
         int64_t zero[MAXD] = {0, 0, 0, 0};
-        HIPCHK(launch_fir1d(src, zero, vo.d, zero, vi.d.n, p, IFM_REPLICATE, 0.f, st));
+        HIPCHK(launch_fir1d(buf, zero, vo.d, zero, vi.d.n, p, IFM_REPLICATE, 0.f, st));
       }
     }
   }

@@ -265,10 +265,13 @@ hipError_t launch_dense_mfma(const Dense4 &in, Dense4 &out, const int64_t *out_f
 hipError_t launch_dense_mfma_batch(int variant, const MfmaArgs *reqs, const int *tile_req, const int *tile_first,
                                    int ntiles, hipStream_t st);
 
-// IIR: one cascade stage along canonical axis `axis`, FP64 recursion.
+// IIR: one cascade stage along canonical axis `axis`, FP64 recursion; in
+// place where in and out are one buffer of one eltype.  out is F64, or any
+// floating-point eltype where the axis length is iir_in_registers.
 struct IirCoef {
   double a[3], b[3], scale, M[9];
 };
+bool iir_in_registers(int64_t n);
 hipError_t launch_iir(const Dense4 &in, Dense4 &out, int axis, const IirCoef &c, int isfill, double fill,
                       hipStream_t st);
 

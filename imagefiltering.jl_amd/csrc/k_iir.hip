@@ -4,20 +4,24 @@
 // (:1027-1048) and rightborder! (:1051-1092): forward recursion with the
 // steady-state left initialisation, right-edge initialisation by the 3x3
 // matrix M (Triggs & Sdika Eqs. 14-15), backward recursion and scaling.
-// Lines of up to 512 elements run k_iir_rows2 (contiguous axis, through an
-// LDS transpose) or k_iir_seg2 (strided axes): whole lines in registers, the
-// axis split into segments, two segments per wave.  Longer lines run
-// k_iir_rows (contiguous axis, LDS-staged chunks) or k_iir_strided (one
-// thread per line).  Lanes sit on adjacent lines, which are adjacent in memory for the
+// Lines of up to 8192 elements run k_iir_line (contiguous axis, through an
+// LDS transpose) or k_iir_seg (strided axes): whole lines in registers, the
+// axis split into segments of one lane each.  Longer lines run k_iir_rows
+// (contiguous axis, LDS-staged chunks) or k_iir_strided (one thread per
+// line).  Lanes sit on adjacent lines, which are adjacent in memory for the
 // strided axes (coalesced).
 #include "ifm_internal.h"
 
 namespace ifm {
 
+#define IFM_GLOBAL __attribute__((address_space(1)))
+
 struct IirArgs {
   const void *src;
-  double *dst;        // FP64 stage result (forward values, then the output)
+  double *dst;        // stage result (the longer lines' kernels also keep forward values there)
   int dt_src;
+  int es_src;         // bytes of a source element
+  int dt_dst;         // F64, or (register-resident lines only) any floating-point eltype
   int n[MAXD];
   int axis;
   int64_t stride;     // element stride of the filtered axis
@@ -255,132 +259,192 @@ __global__ void __launch_bounds__(256, 2) k_iir_rows(IirArgs p) {
   }
 }
 
-// Lines of up to 512 elements, held in registers.  The axis is cut into nw
-// segments of at most IS_S elements, each run by one half-wave lane, so
-// every element is read once and written once (the one-thread-per-line form
-// writes the forward pass out and reads it back).  The recursions are linear:
-// a segment's values are its recursion from zero state plus the homogeneous
+// Lines of up to 8192 elements, held in registers.  The axis is cut into
+// segments of IS_S elements, each run by one lane, so every element is read
+// once and written once (the one-thread-per-line form writes the forward pass
+// out and reads it back, and leaves the chip idle when there are few lines:
+// 3840 x 2160 F32 took 1960 + 292 + 20 us for the two axes and the copy into
+// an F32 output, and takes 71 us this way, of which the bytes are 40).  The
+// recursions are linear: a
+// segment's values are its recursion from zero state plus the homogeneous
 // response to the state entering it.  Each lane runs its segment from zero
-// state; the lanes exchange their end states through LDS; each composes the
-// state entering its segment from those with the 3x3 transfer matrix of a
-// full segment, and adds sum_c h_c[j] s_c.  The first segment's forward pass
-// and the last segment's backward pass start from the reference's border
-// initialisation directly (the um / M start of k_iir_strided).
-constexpr int IS_S = 32;     // most elements per segment (doubles in registers per lane)
-constexpr int IS_MAXW = 16;  // most segments: n <= 512
+// state; the states are then composed along the line (a shuffle scan within
+// the wave, wave totals through LDS), and each lane adds the response to the
+// state entering its segment.  The first segment's forward pass and the last
+// segment's backward pass start from the reference's border initialisation
+// directly (the um / M start of k_iir_strided).
+//
+// A line that does not fill the workgroup's segments is continued before its
+// first element by copies of the value the left border is initialised from
+// (that element, or the Fill value): they keep the recursion in the state it
+// starts in, the steady state of that value, and nothing is stored for them.
+// So every segment has IS_S elements and every loop bound is a constant
+// (bounds per element cost 766 against 652 us on 512 x 512 x 256; a second
+// body for short segments spilled registers: 604 us on 500 x 300 x 200 F64
+// against 275 this way).  What bounds it is HBM on large volumes (512 x 512 x
+// 256 F32 -> F64, three axes: 565 us for 2.95 GB, 5.2 TB/s) and the one
+// load - recursion - store sequence per workgroup on small images.
+constexpr int IS_S = 32;     // elements per segment (doubles in registers per lane)
+constexpr int IS_MAXW = 16;  // most waves per workgroup
+constexpr int IS_MINL = 4;   // fewest lines per workgroup: n <= 64 / 4 * 16 * 32 = 8192
 
 struct IirSegTables {
-  double h[3][IS_S];  // forward homogeneous responses: state (y[-1], y[-2], y[-3]) = e_c
-  double g[3][IS_S];  // backward, by distance from the segment's right end
-  int seg;            // segment length (the last may be shorter, >= 3)
-  int nw;             // segments
+  double pf[5][9];  // forward transfer of a state over 1, 2, 4, 8, 16 segments (row-major 3 x 3)
+  double pb[5][9];  // backward
 };
 
-// LDS (doubles): tables h, g (6 IS_S), then forward and backward end states
-// [segment][component][line] (2 x nw x 3 x 32), then (lines along the
-// contiguous axis) one transpose buffer per wave of 16 rows x IS_TP doubles,
-// which also holds 32 rows x IS_TP floats.
-constexpr int IS_TP = IS_S + 1;    // transpose buffer pitch (elements): conflict-free both ways
-
-// Two segments per wave: a workgroup owns 32 adjacent lines and lane l of
-// wave w runs segment 2w + (l >> 5) of line l & 31.  Segments of at most 32
+// A workgroup owns LN adjacent lines (32, 16, 8 or 4); lane l of wave w runs
+// segment w SPW + l / LN of line l mod LN, SPW = 64 / LN.  Segments of 32
 // elements keep a lane's share of the line in 64 registers, so four waves
-// share each SIMD (two workgroups of up to 8 waves per CU) and one's loads
-// and stores overlap the others' recursions; 64-element segments (two waves
-// per SIMD) measured 942 against 767 us on 512 x 512 x 256.
-//  * k_iir_seg2  strided lines: each half-wave reads one contiguous run of 32
-//                lines per element.
-//  * k_iir_rows2 contiguous lines: a wave's two segments are one run of up
-//                to 64 elements of a line, loaded and stored by its lanes;
-//                they pass through a per-wave LDS transpose (rows = (line,
-//                half) pairs), 16 lines per round for FP32 input, 8 for FP64
-//                input and for the output.
-constexpr int IS_SPW = 2;                 // segments per wave (4, with 16 lines per workgroup, measured slower)
-constexpr int IS2_L = 64 / IS_SPW;        // lines per workgroup
-constexpr int IS2_TB = 16 * IS_TP;        // transpose buffer per wave (doubles)
-__host__ __device__ inline size_t iir_seg2_lds_doubles(int nw, bool rows) {
-  return 6 * IS_S + 2 * (size_t)nw * 3 * IS2_L + (rows ? (size_t)((nw + IS_SPW - 1) / IS_SPW) * IS2_TB : 0);
+// share each SIMD and one's loads and stores overlap the others' recursions;
+// 64-element segments (two waves per SIMD) measured 942 against 767 us on
+// 512 x 512 x 256.
+//  * k_iir_seg   strided lines: lanes of equal segment read LN adjacent
+//                elements.
+//  * k_iir_line  contiguous lines: a wave's segments are one run of SPW * 32
+//                elements of a line, loaded and stored by its lanes; they
+//                pass through a per-wave LDS transpose (rows = (line,
+//                segment) pairs): 32 rows per round for inputs staged as FP32
+//                values, 16 for FP64 input and for the output.  The buffer is
+//                the wave's own, so its rounds need no workgroup barrier.
+constexpr int IS_TP = IS_S + 1;           // transpose buffer pitch (elements): conflict-free both ways
+constexpr int IS_TB = 16 * IS_TP;         // transpose buffer per wave (doubles)
+__host__ __device__ inline size_t iir_seg_lds_doubles(int waves, int ln, bool rows) {
+  return 6 * (size_t)waves * ln + (rows ? (size_t)waves * IS_TB : 0);
 }
 
-struct Seg2 {
-  int ln, sg, L;
-  bool has, first, last;
+struct Seg {
+  int ln, pos, w;  // line and segment of the lane within the wave, wave
+  int at0;         // element of the line the lane's segment starts at (negative: before the line)
+  bool first, last;
 };
 
-__device__ __forceinline__ Seg2 seg2_lane(const IirSegTables &tb, int n) {
-  Seg2 g;
-  const int lane = threadIdx.x & 63;
-  g.ln = lane % IS2_L;
-  g.sg = IS_SPW * (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + lane / IS2_L;
-  g.has = g.sg < tb.nw;
-  g.L = g.has ? min(tb.seg, n - g.sg * tb.seg) : 0;
-  g.first = g.sg == 0;
-  g.last = g.sg == tb.nw - 1;
+template <int LN>
+__device__ __forceinline__ Seg seg_lane(int n) {
+  Seg g;
+  const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+  constexpr int SPW = 64 / LN;
+  g.w = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  g.ln = lane % LN;
+  g.pos = lane / LN;
+  g.at0 = (SPW * g.w + g.pos) * IS_S - (waves * SPW * IS_S - n);
+  g.first = g.w == 0 && g.pos == 0;
+  g.last = g.w == waves - 1 && g.pos == SPW - 1;
   return g;
 }
 
-// The segmented recursion on v[0 .. L) of every lane: forward from zero state (the first segment from leftborder!),
-// end states exchanged through LDS, the homogeneous response of the state
+// LDS writes of this wave are seen by its own later reads.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+struct State3 {
+  double a, b, c;
+};
+
+// s + M t for a 3 x 3 row-major M
+__device__ __forceinline__ State3 st_fma(const double *M, const State3 &t, const State3 &s) {
+  State3 r;
+  r.a = M[0] * t.a + M[1] * t.b + M[2] * t.c + s.a;
+  r.b = M[3] * t.a + M[4] * t.b + M[5] * t.c + s.b;
+  r.c = M[6] * t.a + M[7] * t.b + M[8] * t.c + s.c;
+  return r;
+}
+
+__device__ __forceinline__ State3 st_shfl(const State3 &s, int from) {
+  State3 r;
+  r.a = __shfl(s.a, from);
+  r.b = __shfl(s.b, from);
+  r.c = __shfl(s.c, from);
+  return r;
+}
+
+// The state entering the lane's segment, from the zero-state end states `own`
+// of every segment (the segment the recursion starts in holds its true end
+// state).  REV: the recursion runs from the last segment to the first.  ex:
+// waves x 3 x LN doubles of LDS.  One barrier.
+template <int LN, bool REV>
+__device__ __forceinline__ State3 seg_enter(const double (&pw)[5][9], const Seg &g, State3 own, double *ex) {
+  constexpr int SPW = 64 / LN, KW = SPW == 16 ? 4 : SPW == 8 ? 3 : SPW == 4 ? 2 : 1;
+  const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+  const int at = REV ? SPW - 1 - g.pos : g.pos;    // place in the wave's order
+  const int w = REV ? waves - 1 - g.w : g.w;       // place of the wave
+  const State3 zero = {0.0, 0.0, 0.0};
+#pragma unroll
+  for (int k = 0; k < KW; ++k) {  // inclusive scan within the wave
+    const int d = 1 << k;
+    const State3 o = st_shfl(own, REV ? lane + d * LN : lane - d * LN);
+    if (at >= d) own = st_fma(pw[k], o, own);
+  }
+  if (at == SPW - 1) {
+    ex[(w * 3 + 0) * LN + g.ln] = own.a;
+    ex[(w * 3 + 1) * LN + g.ln] = own.b;
+    ex[(w * 3 + 2) * LN + g.ln] = own.c;
+  }
+  State3 t = st_shfl(own, REV ? lane + LN : lane - LN);
+  if (at == 0) t = zero;
+  __syncthreads();
+  State3 c = zero;                        // state entering the wave
+#pragma unroll 2
+  for (int u = 0; u < w; ++u) {
+    const State3 q = {ex[(u * 3 + 0) * LN + g.ln], ex[(u * 3 + 1) * LN + g.ln], ex[(u * 3 + 2) * LN + g.ln]};
+    c = st_fma(pw[KW], c, q);
+  }
+#pragma unroll
+  for (int k = 0; k < KW; ++k)            // carried over `at` segments
+    if ((at >> k) & 1) c = st_fma(pw[k], c, zero);
+  t.a += c.a;
+  t.b += c.b;
+  t.c += c.c;
+  return t;
+}
+
+// End of one step of a recursion: the steps are not interleaved (the response
+// does not depend on v, and computed ahead it would take 64 more registers).
+__device__ __forceinline__ void step_done(double &v) {
+  asm volatile("" : "+v"(v));
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// The segmented recursion on v of every lane: forward from zero state (the
+// first segment from leftborder!), the homogeneous response of the state
 // entering the segment added; the same backward (the last segment from
-// rightborder!).  Leaves v scaled by nothing; contains two barriers.  FULL:
-// every lane of the wave holds a full segment of IS_S elements (the bounds
-// are then compile-time constants and the per-element predicates vanish).
-template <bool FULL>
-__device__ __forceinline__ void seg2_filter(const IirArgs &p, const IirSegTables &tb, const Seg2 &g, double *sm,
-                                            double (&v)[IS_S]) {
-  double *hs = sm, *gs = sm + 3 * IS_S;
-  double *stf = sm + 6 * IS_S, *stb = stf + tb.nw * 3 * IS2_L;
-  const int nw = tb.nw, S = FULL ? IS_S : tb.seg, L = FULL ? IS_S : g.L, ln = g.ln, sg = g.sg;
-  for (int i = threadIdx.x; i < 6 * IS_S; i += blockDim.x) sm[i] = i < 3 * IS_S ? tb.h[i / IS_S][i % IS_S]
-                                                                                   : tb.g[i / IS_S - 3][i % IS_S];
+// rightborder!).  Leaves v scaled by nothing; contains two barriers.
+template <int LN>
+__device__ __forceinline__ void seg_filter(const IirArgs &p, const IirSegTables &tb, const Seg &g, double *sm,
+                                           double (&v)[IS_S]) {
+  double *stf = sm, *stb = sm + 3 * LN * (blockDim.x >> 6);
   const double a1 = p.a[0], a2 = p.a[1], a3 = p.a[2];
   const double b1 = p.b[0], b2 = p.b[1], b3 = p.b[2];
   const double asum = a1 + a2 + a3, bsum = b1 + b2 + b3;
-  double ym1 = 0.0, ym2 = 0.0, ym3 = 0.0, xlast = 0.0;
-  if (g.first) {
+  double ym1 = 0.0, ym2 = 0.0, ym3 = 0.0;
+  if (g.first) {  // v[0]: the line's first element, or a copy of what the border starts from
     const double iminus = p.isfill ? p.fill : v[0];
     ym1 = ym2 = ym3 = iminus / (1 - asum);
   }
+  const double xlast = v[IS_S - 1];
 #pragma unroll
   for (int j = 0; j < IS_S; ++j) {
-    if (j < L) {
-      if (j == L - 1) xlast = v[j];
-      const double y = v[j] + a1 * ym1 + a2 * ym2 + a3 * ym3;
-      v[j] = y;
-      ym3 = ym2;
-      ym2 = ym1;
-      ym1 = y;
-    }
+    const double y = v[j] + a1 * ym1 + a2 * ym2 + a3 * ym3;
+    v[j] = y;
+    ym3 = ym2;
+    ym2 = ym1;
+    ym1 = y;
+    step_done(v[j]);
   }
-  if (g.has) {
-    stf[(sg * 3 + 0) * IS2_L + ln] = ym1;
-    stf[(sg * 3 + 1) * IS2_L + ln] = ym2;
-    stf[(sg * 3 + 2) * IS2_L + ln] = ym3;
-  }
-  __syncthreads();
-  // state entering segment sg: T_0 = end of segment 0, T_u = Phi T_{u-1} + P_u
-  // with Phi[r][c] = h_c[S - 1 - r]
-  double e0 = ym1, e1 = ym2, e2 = ym3;  // true end state of this segment
-  if (g.has && !g.first) {
-    double t0 = stf[ln], t1 = stf[IS2_L + ln], t2 = stf[2 * IS2_L + ln];
-    for (int u = 1; u < sg; ++u) {
-      const double *q = stf + u * 3 * IS2_L;
-      const double n0 = hs[S - 1] * t0 + hs[IS_S + S - 1] * t1 + hs[2 * IS_S + S - 1] * t2 + q[ln];
-      const double n1 = hs[S - 2] * t0 + hs[IS_S + S - 2] * t1 + hs[2 * IS_S + S - 2] * t2 + q[IS2_L + ln];
-      const double n2 = hs[S - 3] * t0 + hs[IS_S + S - 3] * t1 + hs[2 * IS_S + S - 3] * t2 + q[2 * IS2_L + ln];
-      t0 = n0;
-      t1 = n1;
-      t2 = n2;
-    }
+  State3 r = seg_enter<LN, false>(tb.pf, g, State3{ym1, ym2, ym3}, stf);
 #pragma unroll
-    for (int j = 0; j < IS_S; ++j)
-      if (j < L) v[j] += hs[j] * t0 + hs[IS_S + j] * t1 + hs[2 * IS_S + j] * t2;
-    e0 = ym1 + hs[L - 1] * t0 + hs[IS_S + L - 1] * t1 + hs[2 * IS_S + L - 1] * t2;
-    e1 = ym2 + hs[L - 2] * t0 + hs[IS_S + L - 2] * t1 + hs[2 * IS_S + L - 2] * t2;
-    e2 = ym3 + hs[L - 3] * t0 + hs[IS_S + L - 3] * t1 + hs[2 * IS_S + L - 3] * t2;
+  for (int j = 0; j < IS_S; ++j) {
+    const double y = a1 * r.a + (a2 * r.b + a3 * r.c);
+    v[j] += y;
+    r = State3{y, r.a, r.b};
+    step_done(v[j]);
   }
   double z0 = 0.0, z1 = 0.0, z2 = 0.0;
   if (g.last) {
+    const double e0 = v[IS_S - 1], e1 = v[IS_S - 2], e2 = v[IS_S - 3];
     const double iplus = p.isfill ? p.fill : xlast;
     const double uplus = iplus / (1 - asum);
     const double vplus = uplus / (1 - bsum);
@@ -395,157 +459,244 @@ __device__ __forceinline__ void seg2_filter(const IirArgs &p, const IirSegTables
   double zp1 = 0.0, zp2 = 0.0, zp3 = 0.0;
 #pragma unroll
   for (int j = IS_S - 1; j >= 0; --j) {
-    if (j < L) {
-      double z;
-      if (g.last && j == L - 1) z = z2;
-      else if (g.last && j == L - 2) z = z1;
-      else if (g.last && j == L - 3) z = z0;
-      else z = v[j] + b1 * zp1 + b2 * zp2 + b3 * zp3;
-      v[j] = z;
-      zp3 = zp2;
-      zp2 = zp1;
-      zp1 = z;
-    }
+    double z = v[j] + b1 * zp1 + b2 * zp2 + b3 * zp3;
+    if (j == IS_S - 1) z = g.last ? z2 : z;
+    if (j == IS_S - 2) z = g.last ? z1 : z;
+    if (j == IS_S - 3) z = g.last ? z0 : z;
+    v[j] = z;
+    zp3 = zp2;
+    zp2 = zp1;
+    zp1 = z;
+    step_done(v[j]);
   }
-  if (g.has) {
-    stb[(sg * 3 + 0) * IS2_L + ln] = zp1;
-    stb[(sg * 3 + 1) * IS2_L + ln] = zp2;
-    stb[(sg * 3 + 2) * IS2_L + ln] = zp3;
-  }
-  __syncthreads();
-  // state entering segment sg from the right: R_{nw-1} = left end of the last
-  // segment, R_u = Psi R_{u+1} + Q_u with Psi[r][c] = g_c[S - 1 - r]
-  if (g.has && !g.last) {
-    const double *q0 = stb + (nw - 1) * 3 * IS2_L;
-    double t0 = q0[ln], t1 = q0[IS2_L + ln], t2 = q0[2 * IS2_L + ln];
-    for (int u = nw - 2; u > sg; --u) {
-      const double *q = stb + u * 3 * IS2_L;
-      const double n0 = gs[S - 1] * t0 + gs[IS_S + S - 1] * t1 + gs[2 * IS_S + S - 1] * t2 + q[ln];
-      const double n1 = gs[S - 2] * t0 + gs[IS_S + S - 2] * t1 + gs[2 * IS_S + S - 2] * t2 + q[IS2_L + ln];
-      const double n2 = gs[S - 3] * t0 + gs[IS_S + S - 3] * t1 + gs[2 * IS_S + S - 3] * t2 + q[2 * IS2_L + ln];
-      t0 = n0;
-      t1 = n1;
-      t2 = n2;
-    }
+  r = seg_enter<LN, true>(tb.pb, g, State3{zp1, zp2, zp3}, stb);
 #pragma unroll
-    for (int j = 0; j < IS_S; ++j)
-      if (j < L) v[j] += gs[L - 1 - j] * t0 + gs[IS_S + L - 1 - j] * t1 + gs[2 * IS_S + L - 1 - j] * t2;
+  for (int j = IS_S - 1; j >= 0; --j) {
+    const double z = b1 * r.a + (b2 * r.b + b3 * r.c);
+    v[j] += z;
+    r = State3{z, r.a, r.b};
+    step_done(v[j]);
   }
 }
 
-template <int DT, bool FULL>
-__device__ __forceinline__ void seg2_body(const IirArgs &p, const IirSegTables &tb, const Seg2 &g, double *sm) {
-  const int n = p.n[p.axis];
-  const int L = FULL ? IS_S : g.L;
-  const int64_t line = (int64_t)blockIdx.x * IS2_L + g.ln;
-  const bool ok = line < p.lines && g.has;
-  const int64_t st = p.stride;
-  const int64_t base = (line % st) + (line / st) * st * n + (int64_t)g.sg * tb.seg * st;
-  double v[IS_S];
+// The elements before the line under a Fill border.
+__device__ __forceinline__ void seg_lead(const IirArgs &p, const Seg &g, double (&v)[IS_S]) {
+  if (!p.isfill || g.at0 >= 0) return;
 #pragma unroll
   for (int j = 0; j < IS_S; ++j)
-    if (j < L && ok) v[j] = iir_ld<DT>(p, base + (int64_t)j * st);
-  seg2_filter<FULL>(p, tb, g, sm, v);
-  const double sc = p.scale;
-  if (ok) {
+    if (g.at0 + j < 0) v[j] = p.fill;
+}
+
+// Stage result in the destination eltype: FP64 between the stages, at the
+// last stage whatever the output holds (rounded through FP32 for the 16-bit
+// floats, -0 to +0 as the converting copy rounds).
+template <int DD>  // IFM_F64, IFM_F32, or -1: one of the 16-bit floats
+__device__ __forceinline__ void iir_put(IFM_GLOBAL char *at, int dt, double v) {
+  if constexpr (DD == IFM_F64) *(IFM_GLOBAL double *)at = v;
+  else if constexpr (DD == IFM_F32) *(IFM_GLOBAL float *)at = (float)v + 0.f;
+  else store_f((void *)at, 0, dt, (float)v + 0.f);
+}
+
+// Workgroups of neighbouring lines run on one XCD: with LN < 32 they share
+// cache lines.
+__device__ __forceinline__ int64_t seg_line0(int ln) { return (int64_t)xcd_tile(blockIdx.x, gridDim.x) * ln; }
+
+// Address of element j of a strided line, stepped from element to element:
+// left alone the compiler keeps all 31 multiples of the stride in scalar
+// registers, which spill.
+struct Walk {
+  IFM_GLOBAL char *at;
+  int64_t step;
+  __device__ __forceinline__ Walk(const void *p, int64_t i, int64_t st, int es)
+      : at((IFM_GLOBAL char *)((char *)p + i * es)), step(st * es) {}
+  __device__ __forceinline__ void next(bool more = true) {
+    at += more ? step : 0;
+    asm volatile("" : "+v"(at));
+  }
+};
+
+// FRONT: the wave holds elements before the line.
+template <int DT, bool FRONT>
+__device__ __forceinline__ void seg_load(const IirArgs &p, const Seg &g, int64_t base, double (&v)[IS_S]) {
+  using T = typename std::conditional<DT == IFM_F64, double, float>::type;
+  const int64_t i0 = FRONT ? max(g.at0, 0) : g.at0;
+  Walk q(p.src, base + i0 * p.stride, p.stride, DT == IFM_F32 || DT == IFM_F64 ? (int)sizeof(T) : p.es_src);
 #pragma unroll
-    for (int j = 0; j < IS_S; ++j)
-      if (j < L) p.dst[base + (int64_t)j * st] = v[j] * sc;
+  for (int j = 0; j < IS_S; ++j) {
+    if constexpr (DT == IFM_F32 || DT == IFM_F64) v[j] = (double)*(const IFM_GLOBAL T *)q.at;
+    else v[j] = load_d((const void *)q.at, 0, p.dt_src);
+    q.next(!FRONT || g.at0 + j >= 0);
   }
 }
 
-template <int DT>
-__global__ void __launch_bounds__(32 * IS_MAXW) __attribute__((amdgpu_waves_per_eu(4))) k_iir_seg2(IirArgs p, IirSegTables tb) {
+template <int DD, bool FRONT>
+__device__ __forceinline__ void seg_store(const IirArgs &p, const Seg &g, int64_t base, const double (&v)[IS_S]) {
+  const double sc = p.scale;
+  const int es = DD == IFM_F64 ? 8 : DD == IFM_F32 ? 4 : 2;
+  Walk q(p.dst, base + (int64_t)g.at0 * p.stride, p.stride, es);
+#pragma unroll
+  for (int j = 0; j < IS_S; ++j) {
+    if (!FRONT || g.at0 + j >= 0) iir_put<DD>(q.at, p.dt_dst, v[j] * sc);
+    q.next();
+  }
+}
+
+template <int DT, int LN>
+__global__ void __launch_bounds__(64 * IS_MAXW) __attribute__((amdgpu_waves_per_eu(4))) k_iir_seg(IirArgs p, IirSegTables tb) {
   extern __shared__ double sm[];
-  const Seg2 g = seg2_lane(tb, p.n[p.axis]);
-  // a wave-uniform branch: both bodies pass the same two barriers.  Waves
-  // whose segments all hold 32 elements (every wave when the line length is a
-  // multiple of 32, e.g. 256 or 512) skip the per-element bounds: 766 -> 652
-  // us on the 3-D Gaussian, at four waves per SIMD (128 registers, no spill)
-  if (__all(g.L == IS_S)) seg2_body<DT, true>(p, tb, g, sm);
-  else seg2_body<DT, false>(p, tb, g, sm);
+  const int n = p.n[p.axis];
+  const Seg g = seg_lane<LN>(n);
+  const int64_t ln = seg_line0(LN) + g.ln;
+  const int64_t line = min(ln, p.lines - 1);  // lanes past the last line repeat it and store nothing
+  const int64_t base = (line % p.stride) + (line / p.stride) * p.stride * n;
+  const bool front = __builtin_amdgcn_readfirstlane(g.at0) < 0;  // lane 0 has the wave's first segment
+  double v[IS_S];
+  if (front) seg_load<DT, true>(p, g, base, v);
+  else seg_load<DT, false>(p, g, base, v);
+  seg_lead(p, g, v);
+  seg_filter<LN>(p, tb, g, sm, v);
+  if (ln >= p.lines) return;
+  if (p.dt_dst == IFM_F64) {
+    if (front) seg_store<IFM_F64, true>(p, g, base, v);
+    else seg_store<IFM_F64, false>(p, g, base, v);
+  } else if (p.dt_dst == IFM_F32) {
+    seg_store<IFM_F32, true>(p, g, base, v);
+  } else {
+    seg_store<-1, true>(p, g, base, v);
+  }
 }
 
-template <int DT, bool FULL>
-__device__ __forceinline__ void rows2_body(const IirArgs &p, const IirSegTables &tb, const Seg2 &g, double *sm) {
-  using TE = typename std::conditional<DT == IFM_F32, float, double>::type;
-  const int n = p.n[p.axis];
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63, half = lane / IS2_L;
-  const int S = FULL ? IS_S : tb.seg, nw = tb.nw, L = FULL ? IS_S : g.L;
-  const int64_t line0 = (int64_t)blockIdx.x * IS2_L;
-  double *tr = sm + iir_seg2_lds_doubles(nw, false) + w * IS2_TB;
-  const TE *src = (const TE *)p.src;
-  double v[IS_S];
-  // wave w covers elements [e0, e0 + span) of every line (its two segments);
-  // lane l holds element e0 + l, in transpose row 2 i + l / S, column l % S
-  const int e0 = IS_SPW * w * S, span = min(IS_SPW * S, n - e0);
-  const bool lok = lane < span;
-  const int lh = lane >= S ? 1 : 0, lc = lane - lh * S;
-  constexpr int RI = (DT == IFM_F32 ? 32 : 16) / IS_SPW;  // lines per round
-  TE *tri = (TE *)tr;
-  for (int r = 0; r < IS2_L / RI; ++r) {
-    TE x[RI];
-#pragma unroll
-    for (int i = 0; i < RI; ++i) {
-      const int64_t ln = line0 + r * RI + i;
-      x[i] = (lok && ln < p.lines) ? src[ln * n + e0 + lane] : (TE)0;
-    }
-    if (lok) {
-#pragma unroll
-      for (int i = 0; i < RI; ++i) tri[(IS_SPW * i + lh) * IS_TP + lc] = x[i];
-    }
-    __syncthreads();
-    if ((g.ln / RI) == r) {
-      const int row = (g.ln - r * RI) * IS_SPW + half;
-#pragma unroll
-      for (int j = 0; j < IS_S; ++j)
-        if (j < L) v[j] = (double)tri[row * IS_TP + j];
-    }
-    __syncthreads();
-  }
-  seg2_filter<FULL>(p, tb, g, sm, v);
+// Element as staged: F64 as it is, every other type as FP32 (exact), N0f8 as
+// its code.
+template <int DT>
+__device__ __forceinline__ typename std::conditional<DT == IFM_F64, double, float>::type line_ld(const void *src,
+                                                                                               int64_t i) {
+  if constexpr (DT == IFM_F64) return ((const double *)src)[i];
+  else if constexpr (DT == IFM_F32) return ((const float *)src)[i];
+  else if constexpr (DT == IFM_BF16) return bf16_to_f32(((const uint16_t *)src)[i]);
+  else if constexpr (DT == IFM_F16) return __half2float(((const __half *)src)[i]);
+  else return (float)((const uint8_t *)src)[i];
+}
+
+// Store rounds of the transposed results: RO lines per round.
+template <int DD, int LN>
+__device__ __forceinline__ void line_store(const IirArgs &p, const Seg &g, double *tr, int64_t line0, int w0,
+                                           const double (&v)[IS_S]) {
+  constexpr int SPW = 64 / LN, NC = SPW / 2, RO = 16 / SPW;
+  const int n = p.n[p.axis], lane = threadIdx.x & 63;
+  const int es = DD == IFM_F64 ? 8 : DD == IFM_F32 ? 4 : 2;
   const double sc = p.scale;
-  // stores: rounds of 8 lines (16 rows of doubles)
-  constexpr int RO = 16 / IS_SPW;
-  for (int r = 0; r < IS2_L / RO; ++r) {
+#pragma unroll 1
+  for (int r = 0; r < LN / RO; ++r) {
     if ((g.ln / RO) == r) {
-      const int row = (g.ln - r * RO) * IS_SPW + half;
+      const int row = (g.ln - r * RO) * SPW + g.pos;
 #pragma unroll
-      for (int j = 0; j < IS_S; ++j)
-        if (j < L) tr[row * IS_TP + j] = v[j] * sc;
+      for (int j = 0; j < IS_S; ++j) tr[row * IS_TP + j] = v[j] * sc;
     }
-    __syncthreads();
+    wave_lds_fence();
 #pragma unroll
     for (int i = 0; i < RO; ++i) {
       const int64_t ln = line0 + r * RO + i;
-      if (lok && ln < p.lines) p.dst[ln * n + e0 + lane] = tr[(IS_SPW * i + lh) * IS_TP + lc];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int e = 64 * c + lane;
+        if (w0 + e >= 0 && ln < p.lines)
+          iir_put<DD>((IFM_GLOBAL char *)((char *)p.dst + (ln * n + w0 + e) * es), p.dt_dst,
+                      tr[(SPW * i + e / IS_S) * IS_TP + e % IS_S]);
+      }
     }
-    __syncthreads();
+    wave_lds_fence();
+  }
+}
+
+template <int DT, int LN>
+__global__ void __launch_bounds__(64 * IS_MAXW) __attribute__((amdgpu_waves_per_eu(4))) k_iir_line(IirArgs p, IirSegTables tb) {
+  extern __shared__ double sm[];
+  using TE = typename std::conditional<DT == IFM_F64, double, float>::type;
+  constexpr int SPW = 64 / LN, NC = SPW / 2;           // NC: 64-element loads covering a wave's run of one line
+  constexpr int RI = (DT == IFM_F64 ? 16 : 32) / SPW;  // lines per load round
+  const int n = p.n[p.axis], lane = threadIdx.x & 63;
+  const Seg g = seg_lane<LN>(n);
+  const int w0 = __builtin_amdgcn_readfirstlane(g.at0);  // first element of the wave's run
+  const int64_t line0 = seg_line0(LN);
+  double *tr = sm + iir_seg_lds_doubles(blockDim.x >> 6, LN, false) + g.w * IS_TB;
+  TE *tri = (TE *)tr;
+  double v[IS_S];
+#pragma unroll 1
+  for (int r = 0; r < LN / RI; ++r) {
+    TE x[RI][NC];
+#pragma unroll
+    for (int i = 0; i < RI; ++i) {
+      const int64_t ln = min(line0 + r * RI + i, p.lines - 1);
+#pragma unroll
+      for (int c = 0; c < NC; ++c) x[i][c] = line_ld<DT>(p.src, ln * n + max(w0 + 64 * c + lane, 0));
+    }
+#pragma unroll
+    for (int i = 0; i < RI; ++i)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int e = 64 * c + lane;
+        tri[(SPW * i + e / IS_S) * IS_TP + e % IS_S] = x[i][c];
+      }
+    wave_lds_fence();
+    if ((g.ln / RI) == r) {
+      const int row = (g.ln - r * RI) * SPW + g.pos;
+#pragma unroll
+      for (int j = 0; j < IS_S; ++j)
+        v[j] = DT == IFM_N0F8 ? (double)tri[row * IS_TP + j] / 255.0 : (double)tri[row * IS_TP + j];
+    }
+    wave_lds_fence();
+  }
+  seg_lead(p, g, v);
+  seg_filter<LN>(p, tb, g, sm, v);
+  if (p.dt_dst == IFM_F64) line_store<IFM_F64, LN>(p, g, tr, line0, w0, v);
+  else if (p.dt_dst == IFM_F32) line_store<IFM_F32, LN>(p, g, tr, line0, w0, v);
+  else line_store<-1, LN>(p, g, tr, line0, w0, v);
+}
+
+static int iir_waves(int n, int ln) { return (n + (64 / ln) * IS_S - 1) / ((64 / ln) * IS_S); }
+
+// Lines per workgroup: 32 (the longest runs of adjacent lines) when the
+// segments fit 8 waves, so that two workgroups share a CU, and there are
+// workgroups for every CU; fewer otherwise, but no fewer than 8 while the
+// segments fit 16 waves (200 x 150: 16.9 us with 8, 18.0 with 4; 3840 x 2160:
+// 71 with either).
+static int iir_lines(int n, int64_t lines) {
+  int ln = 32;
+  while (ln > IS_MINL) {
+    const int waves = iir_waves(n, ln);
+    if (waves <= IS_MAXW / 2 && (lines + ln - 1) / ln >= 256) break;
+    if (waves <= IS_MAXW && ln == 8) break;
+    ln /= 2;
+  }
+  return ln;
+}
+
+template <int DT, int LN>
+static void seg_go(const IirArgs &p, const IirSegTables &tb, hipStream_t st) {
+  const int waves = iir_waves(p.n[p.axis], LN);
+  const dim3 grid((unsigned)((p.lines + LN - 1) / LN)), blk(64 * waves);
+  const bool rows = p.stride == 1;
+  const size_t lds = sizeof(double) * iir_seg_lds_doubles(waves, LN, rows);
+  if (rows) {
+    hipLaunchKernelGGL((k_iir_line<DT, LN>), grid, blk, lds, st, p, tb);
+  } else {
+    constexpr int DS = DT == IFM_F32 || DT == IFM_F64 ? DT : -1;  // strided loads of the other types: run-time type
+    hipLaunchKernelGGL((k_iir_seg<DS, LN>), grid, blk, lds, st, p, tb);
   }
 }
 
 template <int DT>
-__global__ void __launch_bounds__(32 * IS_MAXW) __attribute__((amdgpu_waves_per_eu(4))) k_iir_rows2(IirArgs p, IirSegTables tb) {
-  static_assert(DT == IFM_F32 || DT == IFM_F64, "typed contiguous lines only");
-  extern __shared__ double sm[];
-  const Seg2 g = seg2_lane(tb, p.n[p.axis]);
-  // a wave-uniform branch: both bodies pass the same barriers
-  if (__all(g.L == IS_S)) rows2_body<DT, true>(p, tb, g, sm);
-  else rows2_body<DT, false>(p, tb, g, sm);
+static void seg_lines(const IirArgs &p, const IirSegTables &tb, hipStream_t st) {
+  switch (iir_lines(p.n[p.axis], p.lines)) {
+  case 32: seg_go<DT, 32>(p, tb, st); break;
+  case 16: seg_go<DT, 16>(p, tb, st); break;
+  case 8: seg_go<DT, 8>(p, tb, st); break;
+  default: seg_go<DT, 4>(p, tb, st); break;
+  }
 }
 
-// Segmentation of an axis of n elements: nw waves of seg elements (the last
-// one shorter, at least 3); false if n is too long for one workgroup.
-static bool iir_segments(int n, int *seg, int *nw) {
-  const int w = (n + IS_S - 1) / IS_S;
-  if (w > IS_MAXW || n < 4) return false;
-  const int s = (n + w - 1) / w;
-  if (n - (w - 1) * s < 3) return false;
-  *seg = s;
-  *nw = w;
-  return true;
-}
+bool iir_in_registers(int64_t n) { return n >= 4 && n <= (64 / IS_MINL) * IS_MAXW * IS_S; }
 
 hipError_t launch_iir(const Dense4 &in, Dense4 &out, int axis, const IirCoef &c, int isfill, double fill,
                       hipStream_t st) {
@@ -553,6 +704,8 @@ hipError_t launch_iir(const Dense4 &in, Dense4 &out, int axis, const IirCoef &c,
   p.src = in.data;
   p.dst = (double *)out.data;
   p.dt_src = in.dtype;
+  p.es_src = (int)dtype_size(in.dtype);
+  p.dt_dst = out.dtype;
   int64_t stride = 1;
   for (int d = 0; d < MAXD; ++d) {
     p.n[d] = (int)in.n[d];
@@ -570,14 +723,8 @@ hipError_t launch_iir(const Dense4 &in, Dense4 &out, int axis, const IirCoef &c,
   p.isfill = isfill;
   p.fill = fill;
   if (p.lines == 0) return hipSuccess;
-  int seg, nw;
-  const bool typed = in.dtype == IFM_F32 || in.dtype == IFM_F64;
-  // whole lines held in registers (contiguous lines: F32 / F64 input only; the
-  // run-time element type's loads do not fit the transpose rounds' registers)
-  if (iir_segments(p.n[axis], &seg, &nw) && (stride != 1 || typed)) {
+  if (iir_in_registers(in.n[axis])) {  // whole lines held in registers
     IirSegTables tb;
-    tb.seg = seg;
-    tb.nw = nw;
     for (int k = 0; k < 3; ++k) {
       // responses to the unit state e_k: y[-1 - k] = 1
       double hm[3] = {0.0, 0.0, 0.0}, gm[3] = {0.0, 0.0, 0.0};
@@ -585,8 +732,6 @@ hipError_t launch_iir(const Dense4 &in, Dense4 &out, int axis, const IirCoef &c,
       for (int j = 0; j < IS_S; ++j) {
         const double h = c.a[0] * hm[0] + c.a[1] * hm[1] + c.a[2] * hm[2];
         const double g = c.b[0] * gm[0] + c.b[1] * gm[1] + c.b[2] * gm[2];
-        tb.h[k][j] = h;
-        tb.g[k][j] = g;
         hm[2] = hm[1];
         hm[1] = hm[0];
         hm[0] = h;
@@ -594,22 +739,33 @@ hipError_t launch_iir(const Dense4 &in, Dense4 &out, int axis, const IirCoef &c,
         gm[1] = gm[0];
         gm[0] = g;
       }
+      for (int r = 0; r < 3; ++r) {  // the state after one full segment
+        tb.pf[0][3 * r + k] = hm[r];
+        tb.pb[0][3 * r + k] = gm[r];
+      }
     }
-    // two segments per wave, 32 lines per workgroup
-    const bool rows = stride == 1;
-    const unsigned nb2 = (unsigned)((p.lines + IS2_L - 1) / IS2_L);
-    const dim3 blk2(64 * ((nw + IS_SPW - 1) / IS_SPW));
-    const size_t lds2 = sizeof(double) * iir_seg2_lds_doubles(nw, rows);
-    if (rows) {
-      if (in.dtype == IFM_F32) hipLaunchKernelGGL((k_iir_rows2<IFM_F32>), dim3(nb2), blk2, lds2, st, p, tb);
-      else hipLaunchKernelGGL((k_iir_rows2<IFM_F64>), dim3(nb2), blk2, lds2, st, p, tb);
-    } else {
-      if (in.dtype == IFM_F32) hipLaunchKernelGGL((k_iir_seg2<IFM_F32>), dim3(nb2), blk2, lds2, st, p, tb);
-      else if (in.dtype == IFM_F64) hipLaunchKernelGGL((k_iir_seg2<IFM_F64>), dim3(nb2), blk2, lds2, st, p, tb);
-      else hipLaunchKernelGGL((k_iir_seg2<-1>), dim3(nb2), blk2, lds2, st, p, tb);
+    for (int q = 1; q < 5; ++q)
+      for (int r = 0; r < 3; ++r)
+        for (int k = 0; k < 3; ++k) {
+          double f = 0.0, g = 0.0;
+          for (int i = 0; i < 3; ++i) {
+            f += tb.pf[q - 1][3 * r + i] * tb.pf[q - 1][3 * i + k];
+            g += tb.pb[q - 1][3 * r + i] * tb.pb[q - 1][3 * i + k];
+          }
+          tb.pf[q][3 * r + k] = f;
+          tb.pb[q][3 * r + k] = g;
+        }
+    switch (in.dtype) {
+    case IFM_F32: seg_lines<IFM_F32>(p, tb, st); break;
+    case IFM_F64: seg_lines<IFM_F64>(p, tb, st); break;
+    case IFM_BF16: seg_lines<IFM_BF16>(p, tb, st); break;
+    case IFM_F16: seg_lines<IFM_F16>(p, tb, st); break;
+    case IFM_N0F8: seg_lines<IFM_N0F8>(p, tb, st); break;
+    default: seg_lines<IFM_U8>(p, tb, st); break;
     }
     return hipGetLastError();
   }
+  if (out.dtype != IFM_F64) return hipErrorInvalidValue;  // the longer lines' kernels keep forward values in dst
   if (stride == 1) {  // lines along the contiguous axis: LDS-staged chunks
     const unsigned nb = (unsigned)((p.lines + IR_L - 1) / IR_L);
     const size_t lds = sizeof(double) * IR_L * IR_P;

@@ -1090,3 +1090,37 @@ def test_all_finite_device_scan(dtype):
     assert IF.filter_algorithm(IF.DeviceArray.from_host(img), IF.factorkernel(k)) == IF.Algorithm.FIR()
     img[3, 4] = 0.5
     assert IF.filter_algorithm(IF.DeviceArray.from_host(img), IF.factorkernel(k)) == IF.Algorithm.FFT()
+
+
+# ---- IIR lines held in registers ------------------------------------------------------------
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [4, 31, 32, 33, 64, 127, 511, 512, 513, 1025, 2049, 4095, 4097, 8192, 8193])
+@pytest.mark.parametrize("axis", [0, 1])
+def test_iir_line_lengths(n, axis):
+    """Segment counts, lengths that do not fill the segments and the switch to
+    the long-line kernels, over the input and output eltypes and borders.
+
+    Tolerance: each recursion step rounds at 2^-53 of its value and a rounding
+    error is carried on with total weight 1 / (1 - sum a); two passes and their
+    segment composition make fewer than 64 such steps' worth per value.  A
+    Float32 output adds its own rounding."""
+    rng = np.random.default_rng(1000 + 2 * n + axis)
+    other = 37
+    shape = (n, other) if axis == 0 else (other, n)
+    k = IF.KernelFactors.IIRGaussian(4.0)
+    tol = 64 * 2.0 ** -53 / (1 - k.asum)
+    x64 = rng.standard_normal(shape)
+    cases = [(x64, x64), (x64.astype(np.float32), x64.astype(np.float32).astype(np.float64))]
+    codes = rng.integers(0, 256, shape).astype(np.uint8)
+    cases.append((IF.n0f8(codes), codes.astype(np.float64) / 255.0))
+    b16 = IF.bf16(x64)
+    cases.append((b16, IF.bf16_to_float32(b16).astype(np.float64)))
+    for a, ref in cases:
+        a = np.asfortranarray(a).view(type(a))
+        for border, ob in (("replicate", "replicate"), (IF.Fill(1.0), ("fill", 1.0))):
+            want = O.imfilter_iir(np.asfortranarray(ref), [(axis, k.a, k.b, k.scale, k.M)], ob)
+            scale = np.max(np.abs(want))
+            fac = (IF.KernelFactors.ReshapedOneD(2, axis, k),)
+            for T, extra in ((IF.Float64, 0.0), (IF.Float32, 2.0 ** -24)):
+                got = np.asarray(IF.imfilter(T, a, fac, border, IF.Algorithm.IIR()), dtype=np.float64)
+                assert np.max(np.abs(got - want)) <= (tol + extra) * scale, (n, axis, border, T)
