@@ -6,6 +6,8 @@
 //                   generated selection network over a tile of outputs; keys
 //                   of 16 bits or fewer are packed two to a register so each
 //                   v_pk_min_u16 / v_pk_max_u16 serves two tiles.
+//  * k_median_bits  k x k (k = 3 .. 9) centred windows of 8-bit codes on bit
+//                   planes: 32 outputs per VALU instruction.
 //  * k_median_any   any window / border (incl. circular, whose edge windows
 //                   wrap inside the window's intersection with the image,
 //                   src/mapwindow.jl:310-316): counting selection.
@@ -196,6 +198,276 @@ __global__ void __launch_bounds__(256) k_median_net(MedianArgs a) {
                                  tile);
     __syncthreads();
   }
+}
+
+// ---------------------------------------------------------------------------
+// Median of 8-bit codes (UInt8, N0f8) over centred K x K windows, K = 3, 5, 7,
+// 9, on bit planes: a 32-bit word holds one bit of 32 neighbouring pixels, so
+// one VALU instruction serves 32 outputs.  From the highest plane down, the
+// window's bits are counted by a tree of full adders (two v_bitop3 each) and
+// compared with the rank; that is the median's bit.  An element whose bit
+// differs from it is thereby known to lie above or below the median, and goes
+// on counting with the bit it differed in.  K = 7: 8 planes x (42 shifts, 98
+// state updates, 91 adder instructions) / 32 = 55 per output, against 134 of
+// the selection network on keys packed two to a register (k_median_net).
+// Float32 keys would need 32 planes (226 per output against 268 of the
+// network), so the other eltypes keep the network.
+//
+// Tile: 128 x 64 outputs, one word of 32 outputs per thread.  Staging turns 32
+// codes of a row (two unaligned 16-byte loads) into 8 plane words (two 4 x 4
+// byte transposes, one 8 x 8 bit transpose per byte column); results go back
+// the same way and leave through LDS in 16-byte stores.
+// ---------------------------------------------------------------------------
+constexpr int MB_BX = 128, MB_BY = 64;
+constexpr int MB_NW = MB_BX / 32 + 1;  // plane words per staged row (K - 1 <= 32 halo columns)
+
+__device__ __forceinline__ void byte_transpose4(uint32_t &a, uint32_t &b, uint32_t &c, uint32_t &d) {
+  const uint32_t abl = __builtin_amdgcn_perm(b, a, 0x05010400u), abh = __builtin_amdgcn_perm(b, a, 0x07030602u);
+  const uint32_t cdl = __builtin_amdgcn_perm(d, c, 0x05010400u), cdh = __builtin_amdgcn_perm(d, c, 0x07030602u);
+  a = __builtin_amdgcn_perm(cdl, abl, 0x05040100u);
+  b = __builtin_amdgcn_perm(cdl, abl, 0x07060302u);
+  c = __builtin_amdgcn_perm(cdh, abh, 0x05040100u);
+  d = __builtin_amdgcn_perm(cdh, abh, 0x07060302u);
+}
+
+// Bit p of byte q of word i <-> bit i of byte q of word p.
+template <int S>
+__device__ __forceinline__ void bit_swap8(uint32_t (&v)[8]) {
+  constexpr uint32_t m = S == 4 ? 0x0f0f0f0fu : S == 2 ? 0x33333333u : 0x55555555u;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if (i & S) continue;
+    const uint32_t lo = v[i], hi = v[i + S];
+    v[i] = (m & lo) | (~m & (hi << S));
+    v[i + S] = (m & (lo >> S)) | (~m & hi);
+  }
+}
+__device__ __forceinline__ void bit_transpose8(uint32_t (&v)[8]) {
+  bit_swap8<4>(v);
+  bit_swap8<2>(v);
+  bit_swap8<1>(v);
+}
+
+// 32 codes in pixel order (w[i] byte q: pixel 4 i + q) <-> 8 planes (bit j: pixel j).
+__device__ __forceinline__ void codes_to_planes(uint32_t (&w)[8]) {
+  byte_transpose4(w[0], w[2], w[4], w[6]);
+  byte_transpose4(w[1], w[3], w[5], w[7]);
+  uint32_t v[8] = {w[0], w[2], w[4], w[6], w[1], w[3], w[5], w[7]};
+  bit_transpose8(v);
+#pragma unroll
+  for (int p = 0; p < 8; ++p) w[p] = v[p];
+}
+__device__ __forceinline__ void planes_to_codes(uint32_t (&w)[8]) {
+  bit_transpose8(w);
+  byte_transpose4(w[0], w[1], w[2], w[3]);
+  byte_transpose4(w[4], w[5], w[6], w[7]);
+  const uint32_t v[8] = {w[0], w[4], w[1], w[5], w[2], w[6], w[3], w[7]};
+#pragma unroll
+  for (int i = 0; i < 8; ++i) w[i] = v[i];
+}
+
+// Per bit position, whether at least 2^BITS - C of N inputs are set, as they
+// arrive: the I-th input of a weight waits (s, t) until a full adder can take
+// three; the sum stays, the carry is an input of the next weight.  Taken in
+// this order few partial sums are live at once (128 registers instead of 159
+// for K = 7).  N is odd at every weight; a constant bit of C turns the last
+// sum of its weight into one more carry.
+template <int N, int C, int BITS>
+struct RankCounter {
+  static_assert(N % 2 == 1 && N >= 3, "odd count");
+  uint32_t s, t;
+  RankCounter<(N - 1) / 2 + (C & 1), C / 2, BITS - 1> up;
+  template <int I>  // I = 1 .. N
+  __device__ __forceinline__ void add(uint32_t x) {
+    if constexpr (I == 1) {
+      s = x;
+    } else if constexpr (I % 2 == 0) {
+      t = x;
+    } else {
+      const uint32_t carry = __builtin_amdgcn_bitop3_b32(s, t, x, 0xe8);
+      s = __builtin_amdgcn_bitop3_b32(s, t, x, 0x96);
+      up.template add<(I - 1) / 2>(carry);
+    }
+    if constexpr (I == N && (C & 1)) up.template add<(N - 1) / 2 + 1>(s);
+  }
+  __device__ __forceinline__ uint32_t result() const { return up.result(); }
+};
+template <int N>
+struct RankCounter<N, 0, 1> {
+  static_assert(N == 3, "three bits of half the bound's weight");
+  uint32_t s, t;
+  template <int I>
+  __device__ __forceinline__ void add(uint32_t x) {
+    if constexpr (I == 1) s = x;
+    else if constexpr (I == 2) t = x;
+    else s = __builtin_amdgcn_bitop3_b32(s, t, x, 0xe8);
+  }
+  __device__ __forceinline__ uint32_t result() const { return s; }
+};
+
+template <int K>
+struct BitRank {
+  static constexpr int L = K * K;
+  static constexpr int BITS = K == 3 ? 3 : K == 5 ? 4 : K == 7 ? 5 : 6;
+  static constexpr int C = (1 << BITS) - (L + 1) / 2;  // bit 1 iff set bits + C >= 2^BITS
+  using Counter = RankCounter<L, C, BITS>;
+};
+
+// Element I (row I / K) of the window on one plane: its bit is counted, and
+// kept in `last` for the next plane's state.
+template <int K, int I>
+__device__ __forceinline__ void bits_element(const uint32_t *src, uint32_t &lo, uint32_t &hi,
+                                             const uint32_t (&known)[K * K], uint32_t (&last)[K * K],
+                                             typename BitRank<K>::Counter &n) {
+  if constexpr (I % K == 0) {
+    lo = src[(I / K) * MB_NW];
+    hi = src[(I / K) * MB_NW + 1];
+  }
+  const uint32_t b = I % K ? __builtin_amdgcn_alignbit(hi, lo, I % K) : lo;
+  last[I] = (known[I] & last[I]) | (~known[I] & b);
+  n.template add<I + 1>(last[I]);
+  if constexpr (I + 1 < K * K) bits_element<K, I + 1>(src, lo, hi, known, last, n);
+}
+
+template <int K>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(K == 9 ? 2 : 4))) k_median_bits(MedianArgs a) {
+  constexpr int LH = MB_BY + K - 1, H = K / 2, L = K * K;
+  constexpr int RW = MB_NW * 32;      // staged columns
+  constexpr int PP = LH * MB_NW + 1;  // plane pitch (words)
+  static_assert(LH + RW <= 256, "one table entry per thread");
+  __shared__ uint32_t planes[8 * PP];
+  __shared__ uint4 codes[LH * RW / 16];  // staged codes of a border tile, then the results
+  __shared__ int rows[LH];               // border-mapped image row / column of each staged one, -1: Fill
+  __shared__ int4 cols[RW / 4];
+  const int tid = threadIdx.x;
+  // tiles XCD by XCD: row neighbours share their halo columns' cache lines
+  const int tile = xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
+  const int bx = (tile % gridDim.x) * MB_BX, by = (tile / gridDim.x) * MB_BY;
+  const int gx = a.f0 + bx - H, gy = a.f1 + by - H;
+  const bool inside = gx >= 0 && gx + RW <= a.n0;  // every staged column is an image column
+  {
+    const bool isrow = tid < LH;
+    const int at = bmap(a.style, isrow ? gy + tid : gx + tid - LH, isrow ? a.n1 : a.n0);
+    if (isrow) rows[tid] = at;
+    else if (tid < LH + RW) ((int *)cols)[tid - LH] = at;
+  }
+  __syncthreads();
+  for (int plane = blockIdx.z; plane < a.nplanes; plane += gridDim.z) {
+    const int p2 = plane % a.o2, p3 = plane / a.o2;
+    const uint8_t *in = (const uint8_t *)a.in + ((int64_t)(p2 + a.f2) + (int64_t)a.n2 * (p3 + a.f3)) * a.in_plane;
+    const int64_t obase = (int64_t)plane * a.out_plane;
+    if (!inside) {  // four codes of a row per thread and step, 16 loads in flight
+      constexpr int WR = RW / 4, NB = 4;
+#pragma unroll 1
+      for (int e0 = tid; e0 < LH * WR; e0 += 256 * NB) {
+        uint8_t k[NB][4];
+        int4 c[NB];
+        int sy[NB];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+          const int e = min(e0 + 256 * i, LH * WR - 1), r = e / WR;
+          sy[i] = rows[r];
+          c[i] = cols[e - r * WR];
+          const uint8_t *row = in + (int64_t)max(sy[i], 0) * a.n0;
+          k[i][0] = row[max(c[i].x, 0)];
+          k[i][1] = row[max(c[i].y, 0)];
+          k[i][2] = row[max(c[i].z, 0)];
+          k[i][3] = row[max(c[i].w, 0)];
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+          const uint32_t f = a.fillkey;
+          uint32_t x = (c[i].x | sy[i]) < 0 ? f : k[i][0];
+          x |= ((c[i].y | sy[i]) < 0 ? f : k[i][1]) << 8;
+          x |= ((c[i].z | sy[i]) < 0 ? f : k[i][2]) << 16;
+          x |= ((c[i].w | sy[i]) < 0 ? f : k[i][3]) << 24;
+          if (e0 + 256 * i < LH * WR) ((uint32_t *)codes)[e0 + 256 * i] = x;
+        }
+      }
+      __syncthreads();
+    }
+#pragma unroll 1
+    for (int item = tid; item < LH * MB_NW; item += 256) {
+      const int r = item / MB_NW, cw = item - r * MB_NW;
+      uint32_t w[8];
+      if (inside) {
+        const int sy = rows[r];
+        __builtin_memcpy(w, in + (int64_t)max(sy, 0) * a.n0 + gx + 32 * cw, 32);
+        if (sy < 0) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) w[i] = a.fillkey * 0x01010101u;
+        }
+      } else {
+        const uint4 x = codes[2 * item], y = codes[2 * item + 1];
+        w[0] = x.x, w[1] = x.y, w[2] = x.z, w[3] = x.w;
+        w[4] = y.x, w[5] = y.y, w[6] = y.z, w[7] = y.w;
+      }
+      codes_to_planes(w);
+#pragma unroll
+      for (int p = 0; p < 8; ++p) planes[p * PP + item] = w[p];
+    }
+    __syncthreads();
+    {
+      const int xw = tid & (MB_BX / 32 - 1), y = tid / (MB_BX / 32);
+      uint32_t known[L], last[L];  // elements known to differ from the median, and their bit
+#pragma unroll
+      for (int i = 0; i < L; ++i) known[i] = last[i] = 0;
+      uint32_t *res = (uint32_t *)(codes + 2 * tid);
+#pragma unroll 1
+      for (int p = 7; p >= 0; --p) {
+        typename BitRank<K>::Counter n;
+        uint32_t lo, hi;
+        bits_element<K, 0>(planes + p * PP + y * MB_NW + xw, lo, hi, known, last, n);
+        const uint32_t m = n.result();
+        res[p] = m;
+#pragma unroll
+        for (int i = 0; i < L; ++i) known[i] = __builtin_amdgcn_bitop3_b32(known[i], last[i], m, 0xf6);
+      }
+      uint32_t m[8];
+#pragma unroll
+      for (int p = 0; p < 8; ++p) m[p] = res[p];
+      planes_to_codes(m);
+      codes[2 * tid] = make_uint4(m[0], m[1], m[2], m[3]);
+      codes[2 * tid + 1] = make_uint4(m[4], m[5], m[6], m[7]);
+    }
+    __syncthreads();
+    if (a.odt == a.dt) {  // 16 codes per store, at any alignment
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int i = tid + 256 * k, oy = by + i / (MB_BX / 16), ox = bx + 16 * (i % (MB_BX / 16));
+        if (oy >= a.o1) continue;
+        uint8_t *dst = (uint8_t *)a.out + obase + (int64_t)oy * a.o0 + ox;
+        if (ox + 16 <= a.o0) {
+          __builtin_memcpy(dst, &codes[i], 16);
+        } else {
+          for (int b = 0; ox + b < a.o0; ++b) dst[b] = ((const uint8_t *)&codes[i])[b];
+        }
+      }
+    } else {
+      const uint8_t *c = (const uint8_t *)codes + tid;
+      const int ox = bx + (tid & (MB_BX - 1)), oy0 = by + tid / MB_BX;
+      const int nr = ox < a.o0 ? min((a.o1 - oy0 + 1) / 2, MB_BY / 2) : 0;  // rows oy0, oy0 + 2, ...
+      const int64_t o = obase + (int64_t)oy0 * a.o0 + ox;
+      const bool n0f8 = a.dt == IFM_N0F8;
+      if (a.odt == IFM_F32) {
+        float *dst = (float *)a.out + o;
+#pragma unroll 4
+        for (int r = 0; r < nr; ++r, dst += 2 * a.o0) *dst = n0f8 ? n0f8_to_f32(c[256 * r]) : (float)c[256 * r];
+      } else {
+        double *dst = (double *)a.out + o;
+#pragma unroll 4
+        for (int r = 0; r < nr; ++r, dst += 2 * a.o0)
+          *dst = n0f8 ? (double)c[256 * r] / 255.0 : (double)c[256 * r];
+      }
+    }
+    __syncthreads();
+  }
+}
+
+template <int K>
+static void launch_bits(const MedianArgs &a, hipStream_t st) {
+  dim3 grid((a.o0 + MB_BX - 1) / MB_BX, (a.o1 + MB_BY - 1) / MB_BY, a.nplanes < 65535 ? a.nplanes : 65535);
+  hipLaunchKernelGGL(k_median_bits<K>, grid, dim3(256), 0, st, a);
 }
 
 // Batched serving: tile g belongs to request tile_req[g]; its requests are
@@ -548,6 +820,18 @@ hipError_t launch_median_band_batch(int k, const BandJob *jobs, const int *tile_
   return hipGetLastError();
 }
 
+// Bit planes or selection network for codes.  One bit-plane tile takes longer
+// than one network tile (its 8 planes are a serial chain), so below about one
+// tile per CU the network is faster for K = 5 and 7: 1024^2 (128 tiles) 6.7 /
+// 9.3 us against 8.5 / 11.3; 1448^2 (276 tiles) 10.9 / 18.0 against 9.8 /
+// 13.2; 8192^2 162 / 326 against 75 / 123.  K = 3: 724^2 8.5 against 6.6,
+// 8192^2 109 against 51.
+static bool median_on_bits(const MedianArgs &a, bool codes, int k) {
+  if (!codes || a.fillkey > 0xffu) return false;
+  const int64_t tiles = (int64_t)((a.o0 + MB_BX - 1) / MB_BX) * ((a.o1 + MB_BY - 1) / MB_BY) * a.nplanes;
+  return k == 3 || k == 9 || tiles >= 192;
+}
+
 hipError_t launch_median(const Dense4 &in, Dense4 &out, const int64_t *out_first, const int *wfirst,
                          const int *wlen, int style, double fill, hipStream_t st) {
   if (out.count() == 0) return hipSuccess;
@@ -555,10 +839,12 @@ hipError_t launch_median(const Dense4 &in, Dense4 &out, const int64_t *out_first
   // image-relative border map equals mapwindow's window-relative one for such
   // windows except for circular, whose edge band is recomputed afterwards.
   int k = wlen[0];
-  bool square = (k == 3 || k == 5 || k == 7) && wlen[1] == k && wfirst[0] == -(k / 2) && wfirst[1] == -(k / 2) &&
+  const bool codes = in.dtype == IFM_U8 || in.dtype == IFM_N0F8;
+  const bool nine = k == 9 && codes && style != IFM_CIRCULAR;  // the circular edge band is for k <= 7
+  bool square = (k == 3 || k == 5 || k == 7 || nine) && wlen[1] == k && wfirst[0] == -(k / 2) && wfirst[1] == -(k / 2) &&
                 wlen[2] == 1 && wlen[3] == 1 && wfirst[2] == 0 && wfirst[3] == 0;
   bool small = in.n[0] >= k && in.n[1] >= k;  // mirrored maps stay within the window
-  if (square && small && in.dtype != IFM_F64) {
+  if (square && small && in.dtype != IFM_F64 && !(nine && fill_key32(in.dtype, fill) > 0xffu)) {
     MedianArgs a;
     a.in = in.data;
     a.out = out.data;
@@ -580,7 +866,12 @@ hipError_t launch_median(const Dense4 &in, Dense4 &out, const int64_t *out_first
     a.odt = out.dtype;
     a.fillkey = fill_key32(in.dtype, fill);
     bool pack = in.dtype != IFM_F32;
-    if (k == 3) {
+    if (median_on_bits(a, codes, k)) {
+      if (k == 3) launch_bits<3>(a, st);
+      else if (k == 5) launch_bits<5>(a, st);
+      else if (k == 7) launch_bits<7>(a, st);
+      else launch_bits<9>(a, st);
+    } else if (k == 3) {
       if (pack) launch_net_on<3, 4, 2, 2>(a, st); else launch_net_on<3, 4, 2, 1>(a, st);
     } else if (k == 5) {
       if (pack) launch_net_on<5, 2, 2, 2>(a, st); else launch_net_on<5, 2, 2, 1>(a, st);

@@ -1093,7 +1093,6 @@ def test_all_finite_device_scan(dtype):
 
 
 # ---- IIR lines held in registers ------------------------------------------------------------
-@pytest.mark.gpu
 @pytest.mark.parametrize("n", [4, 31, 32, 33, 64, 127, 511, 512, 513, 1025, 2049, 4095, 4097, 8192, 8193])
 @pytest.mark.parametrize("axis", [0, 1])
 def test_iir_line_lengths(n, axis):
@@ -1124,3 +1123,42 @@ def test_iir_line_lengths(n, axis):
             for T, extra in ((IF.Float64, 0.0), (IF.Float32, 2.0 ** -24)):
                 got = np.asarray(IF.imfilter(T, a, fac, border, IF.Algorithm.IIR()), dtype=np.float64)
                 assert np.max(np.abs(got - want)) <= (tol + extra) * scale, (n, axis, border, T)
+
+
+# ---- medians on bit planes -------------------------------------------------------------------
+@pytest.mark.parametrize("k", [3, 5, 7, 9])
+@pytest.mark.parametrize("shape", [(9, 9), (31, 64), (127, 63), (128, 65), (129, 64), (163, 130), (288, 33)])
+def test_median_codes_tile_edges(k, shape):
+    """Tile and word edges of the bit-plane median (128 x 64 tiles, words of 32
+    columns) on enough planes for it to be taken (192 tiles), every border,
+    code and Float32 results, an Inner() interior: bit-exact."""
+    from imagefiltering import _lib
+    from imagefiltering.device import ifm_array
+    rng = np.random.default_rng(k * 1000 + shape[0])
+    h = k // 2
+    tiles = -(-(shape[0] - 2 * h) // 128) * -(-(shape[1] - 2 * h) // 64)
+    planes = -(-192 // max(tiles, 1))
+    vol = rng.integers(0, 256, shape + (planes,)).astype(np.uint8)
+    vol[:, :, ::2] %= 3                                  # ties
+    vol = np.asfortranarray(vol)
+    some = [0, 1, planes - 1]
+    for b in STYLES + [IF.Fill(7)]:
+        got = np.asarray(IF.mapwindow(IF.median_, vol, (k, k, 1), border=b))
+        for z in some:
+            want = O.median(vol[:, :, z].astype(np.float64), [-h, -h], [k, k], obord(b))
+            np.testing.assert_array_equal(got[:, :, z], want)
+    gotf = np.asarray(IF.mapwindow(IF.median_, IF.n0f8(vol), (k, k, 1), border="reflect"))
+    d = IF.DeviceArray.from_host(vol)
+    out = d.similar()
+    bs = _lib.IfmBorder()
+    bs.style = _lib.REFLECT
+    _lib.check(_lib.load().ifm_mapwindow_median(_lib.ctx(), ifm_array(d), ifm_array(out), None,
+                                                _lib.i64([-h, -h, 0]), _lib.i64([k, k, 1], 1), bs))
+    codes = out.to_host()
+    inner = IF.mapwindow(IF.median_, vol, (k, k, 1), border=IF.Inner()).data if min(shape) > k else None
+    for z in some:
+        want = O.median(vol[:, :, z].astype(np.float64), [-h, -h], [k, k], "reflect")
+        np.testing.assert_array_equal(codes[:, :, z], want)
+        np.testing.assert_array_equal(gotf[:, :, z], (want / 255).astype(np.float32))
+        if inner is not None:
+            np.testing.assert_array_equal(np.asarray(inner)[:, :, z], want[h:shape[0] - h, h:shape[1] - h])
