@@ -1162,3 +1162,42 @@ def test_median_codes_tile_edges(k, shape):
         np.testing.assert_array_equal(gotf[:, :, z], (want / 255).astype(np.float32))
         if inner is not None:
             np.testing.assert_array_equal(np.asarray(inner)[:, :, z], want[h:shape[0] - h, h:shape[1] - h])
+
+
+# ---- Float64 medians and 9 x 9 windows ---------------------------------------------------------
+@pytest.mark.parametrize("k", [3, 5, 7, 9])
+@pytest.mark.parametrize("shape", [(9, 9), (63, 17), (65, 16), (129, 33)])
+def test_median_float64_networks(k, shape):
+    """The networks on Float64 values and the 9 x 9 network of the other float
+    eltypes: tile edges, borders, ties, signed zeros, infinities and NaN (from a
+    few to whole windows), an Inner() interior.  Bit-exact, signs of zero included."""
+    rng = np.random.default_rng(7 * k + shape[0])
+    h = k // 2
+    base = np.asfortranarray(rng.integers(-2, 3, shape) * rng.integers(0, 2, shape) * 1.0)
+    base[base == 0] *= np.where(rng.random(int(np.sum(base == 0))) < 0.5, -1.0, 1.0)
+    fine = np.asfortranarray(rng.standard_normal(shape))
+    bad = fine.copy(order="F")
+    bad[rng.random(shape) < 0.02] = np.inf
+    bad[rng.random(shape) < 0.02] = -np.inf
+    bad[rng.random(shape) < 0.05] = np.nan
+    bad[: 2 * h + 1, : k] = np.nan
+    for img in (base, fine, bad):
+        for b in STYLES + [IF.Fill(0.5), IF.Fill(float("nan"))]:
+            want = O.median(img, [-h, -h], [k, k], obord(b))
+            got = np.asarray(IF.mapwindow(IF.median_, img, (k, k), border=b))
+            np.testing.assert_array_equal(got, want)
+            np.testing.assert_array_equal(np.signbit(got[want == 0]), np.signbit(want[want == 0]))
+        if min(shape) > k:
+            want = O.median(img, [-h, -h], [k, k], "replicate")
+            got = IF.mapwindow(IF.median_, img, (k, k), border=IF.Inner()).data
+            np.testing.assert_array_equal(got, want[h:shape[0] - h, h:shape[1] - h])
+        if k == 9:
+            for b in ("replicate", "reflect", "circular"):
+                f = img.astype(np.float32)
+                want = O.median(f.astype(np.float64), [-h, -h], [k, k], b)
+                np.testing.assert_array_equal(IF.mapwindow(IF.median_, f, (k, k), border=b), want)
+                x = IF.bf16(img)
+                xv = IF.bf16_to_float32(x)
+                want = O.median(xv.astype(np.float64), [-h, -h], [k, k], b)
+                got = IF.mapwindow(IF.median_, np.asfortranarray(x).view(IF.BF16Array), (k, k), border=b)
+                np.testing.assert_array_equal(IF.bf16_to_float32(got), want.astype(np.float32))
