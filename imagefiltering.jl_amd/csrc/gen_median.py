@@ -219,7 +219,8 @@ def emit(net, outs, k, tx, ty):
                              k, tx, ty, cols * rows, tx * ty, body, rets))
 
 
-CONFIGS = [(3, 4, 2, 2), (5, 2, 2, 1), (7, 2, 2, 1), (9, 2, 2, 1)]  # k, tx, ty, selection mode
+CONFIGS = [(3, 4, 2, 2), (5, 2, 2, 1), (7, 2, 2, 1), (9, 2, 2, 1),
+           (3, 1, 1, 2), (5, 1, 1, 1), (7, 1, 1, 1)]  # k, tx, ty, selection mode
 
 if __name__ == "__main__":
     if len(sys.argv) > 1 and sys.argv[1] == "--survey":

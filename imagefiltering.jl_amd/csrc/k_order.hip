@@ -55,6 +55,16 @@ template <> struct MedianNet<9, 2, 2> {
   template <typename T> static __device__ __forceinline__ void run(const T (&v)[100], T (&o)[4]) { median_net_9_2_2(v, o); }
 };
 
+template <> struct MedianNet<3, 1, 1> {
+  template <typename T> static __device__ __forceinline__ void run(const T (&v)[9], T (&o)[1]) { median_net_3_1_1(v, o); }
+};
+template <> struct MedianNet<5, 1, 1> {
+  template <typename T> static __device__ __forceinline__ void run(const T (&v)[25], T (&o)[1]) { median_net_5_1_1(v, o); }
+};
+template <> struct MedianNet<7, 1, 1> {
+  template <typename T> static __device__ __forceinline__ void run(const T (&v)[49], T (&o)[1]) { median_net_7_1_1(v, o); }
+};
+
 // Block = TXT x TYT threads (32 x 8, or 16 x 16 where 32 columns of threads
 // would stage more than 128 columns); thread tile TX x TY outputs, PACK tiles
 // stacked in rows (PACK = 2 packs two 16-bit keys per register).
@@ -808,7 +818,17 @@ static hipError_t median_any_region(const Dense4 &in, Dense4 &out, const int64_t
 // the image are recomputed after the network kernel has written every output
 // (the interior is style-independent).  One thread per band output gathers
 // its k*k keys into registers through the window-relative map and selects the
-// ((L+1)÷2)-th smallest by counting.
+// ((L+1)÷2)-th smallest by a network of its own (7 x 7: 570 operations; by
+// counting 7,200, 43 us of a 24-request batch).
+template <int K, int DT>
+__device__ __forceinline__ void band_keys(const void *in, const int64_t (&row)[K], const int (&x)[K],
+                                          uint32_t (&k)[K * K]) {
+#pragma unroll
+  for (int v = 0; v < K; ++v)
+#pragma unroll
+    for (int u = 0; u < K; ++u) k[v * K + u] = key_of<DT>(in, row[v] + x[u]);
+}
+
 template <int K>
 __device__ __forceinline__ void band_one(const BandJob &j, int local, int plane) {
   constexpr int H = K / 2, L = K * K;
@@ -818,31 +838,29 @@ __device__ __forceinline__ void band_one(const BandJob &j, int local, int plane)
   const int xlo = max(0, x - H), xm = min(j.n0 - 1, x + H) - xlo + 1;
   const int ylo = max(0, y - H), ym = min(j.n1 - 1, y + H) - ylo + 1;
   const int64_t ibase = (int64_t)plane * j.in_plane;
-  uint32_t k[L];
+  int xx[K];
+#pragma unroll
+  for (int u = 0; u < K; ++u) {
+    xx[u] = x - H + u;
+    if (xx[u] < xlo || xx[u] >= xlo + xm) xx[u] = xlo + imod(xx[u] - xlo, xm);
+  }
+  int64_t row[K];
 #pragma unroll
   for (int v = 0; v < K; ++v) {
     int yy = y - H + v;
     if (yy < ylo || yy >= ylo + ym) yy = ylo + imod(yy - ylo, ym);
-#pragma unroll
-    for (int u = 0; u < K; ++u) {
-      int xx = x - H + u;
-      if (xx < xlo || xx >= xlo + xm) xx = xlo + imod(xx - xlo, xm);
-      k[v * K + u] = key32(j.in, ibase + (int64_t)yy * j.n0 + xx, j.dt);
-    }
+    row[v] = ibase + (int64_t)yy * j.n0;
   }
-  constexpr int rank = (L + 1) / 2 - 1;
-  uint32_t res = k[0];
-#pragma unroll
-  for (int i = 0; i < L; ++i) {
-    int less = 0, eq = 0;
-#pragma unroll
-    for (int t = 0; t < L; ++t) {
-      less += k[t] < k[i];
-      eq += k[t] == k[i];
-    }
-    res = (less <= rank && rank < less + eq) ? k[i] : res;
+  uint32_t k[L], res[1];
+  switch (j.dt) {  // one choice for all loads, so that they are in flight together
+  case IFM_U8:
+  case IFM_N0F8: band_keys<K, IFM_U8>(j.in, row, xx, k); break;
+  case IFM_F32: band_keys<K, IFM_F32>(j.in, row, xx, k); break;
+  case IFM_BF16: band_keys<K, IFM_BF16>(j.in, row, xx, k); break;
+  default: band_keys<K, IFM_F16>(j.in, row, xx, k); break;
   }
-  store_key_as(j.out, (int64_t)plane * j.out_plane + (int64_t)oy * j.opitch + ox, j.dt, j.odt, res);
+  MedianNet<K, 1, 1>::run(k, res);
+  store_key_as(j.out, (int64_t)plane * j.out_plane + (int64_t)oy * j.opitch + ox, j.dt, j.odt, res[0]);
 }
 
 struct BandJobs4 {
