@@ -49,6 +49,14 @@ __device__ __forceinline__ int xcd_tile(int lin, int n) {
   return x * per + min(x, rem) + k;
 }
 
+// LDS writes of this wave are seen by its own later reads, and follow its
+// earlier ones (LDS serves a wave in order; this keeps the compiler to it).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // N0f8 code / 255 rounded to nearest (Float32(x::N0f8)): the product with the
 // rounded reciprocal corrected by one FMA step, which equals the correctly
 // rounded quotient for every code 0..255 (checked exhaustively on the CPU).
@@ -369,8 +377,14 @@ struct SepReq {
   int k0, k1, first0, first1;
   int style, dt_in, dt_out;
   float fill;
-  int ty;  // tile height (S2_TY or S2_TY2)
+  int ty;  // tile height (S2_TY or S2_TY2), or rows per chunk of a marched request
 };
+// Whether a pair of factors can be marched (sep_march), and the workgroups and
+// rows per chunk of a marched request.
+bool sep_march_takes(int k0, int k1, int dt_in);
+int sep_march_groups(int n0, int n1, int *rows);
+hipError_t launch_sep_march_batch(const SepReq *reqs, const int *tile_req, const int *tile_first, int ntiles,
+                                  hipStream_t st);
 hipError_t launch_sep_batch(const SepReq *reqs, const int *tile_req, const int *tile_first, int ntiles,
                             size_t lds_bytes, hipStream_t st);
 void median_batch_tile(int k, bool pack, int *bx, int *by);

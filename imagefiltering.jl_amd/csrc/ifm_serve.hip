@@ -218,7 +218,7 @@ DenseKernel dense_of(const ifm_kernel &k) {
 // Launch list of one batch, with offsets into the descriptor block.
 struct Group {
   int kind;     // 0 fill, 1 separable, 2 median, 3 dense, 4 circular median band, 5 Toeplitz tables
-  int param;    // median: k * 2 + pack; dense: variant
+  int param;    // separable: marched; median: k * 2 + pack; dense: variant
   size_t reqs, tile_req, tile_first;
   int ntiles;
   size_t lds;
@@ -272,8 +272,9 @@ int build_batch(ifm_ctx *ctx, const ifm_request *reqs, const int *idx, int n, co
     }
     if (!fr.empty()) tiles_group(0, 0, mem, nt, blk.put(fr.data(), fr.size() * sizeof(FillReq)), 0);
   }
-  // Separable.
-  {
+  // Separable: the marched requests and the ones in tiles.  A batch has rows
+  // enough to fill the chip by marching, whatever its images' sizes.
+  for (int marched = 0; marched < 2; ++marched) {
     std::vector<int> mem, nt;
     std::vector<SepReq> sr;
     std::vector<std::pair<size_t, size_t>> tapoffs;  // (offset of taps0, taps1)
@@ -312,12 +313,19 @@ int build_batch(ifm_ctx *ctx, const ifm_request *reqs, const int *idx, int n, co
       s.dt_in = vin[i].dtype;
       s.dt_out = part ? q.out2.dtype : vout[i].dtype;
       s.fill = (float)q.border.fill;
-      s.ty = sep2d_tile_h(ctx, s.dt_in, k0, k1, (int64_t)s.n0 * s.n1);
+      if ((int)sep_march_takes(k0, k1, s.dt_in) != marched) continue;
+      int tiles;
+      if (marched) {
+        tiles = sep_march_groups(s.n0, s.n1, &s.ty);
+      } else {
+        s.ty = sep2d_tile_h(ctx, s.dt_in, k0, k1, (int64_t)s.n0 * s.n1);
+        lds = std::max(lds, sizeof(float) * sep2d_lds_floats(k0, k1, s.ty));
+        tiles = ((s.n0 + S2_TX - 1) / S2_TX) * ((s.n1 + s.ty - 1) / s.ty);
+      }
       sr.push_back(s);
       tapoffs.push_back({blk.put(t0, sizeof(float) * k0, 16), blk.put(t1, sizeof(float) * k1, 16)});
-      lds = std::max(lds, sizeof(float) * sep2d_lds_floats(k0, k1, s.ty));
       mem.push_back(i);
-      nt.push_back((int)(((s.n0 + S2_TX - 1) / S2_TX) * ((s.n1 + s.ty - 1) / s.ty)));
+      nt.push_back(tiles);
     }
     if (!sr.empty()) {
       size_t off = blk.put(sr.data(), sr.size() * sizeof(SepReq));
@@ -325,7 +333,7 @@ int build_batch(ifm_ctx *ctx, const ifm_request *reqs, const int *idx, int n, co
         blk.ptr(off + m * sizeof(SepReq) + offsetof(SepReq, taps0), tapoffs[m].first);
         blk.ptr(off + m * sizeof(SepReq) + offsetof(SepReq, taps1), tapoffs[m].second);
       }
-      tiles_group(1, 0, mem, nt, off, lds);
+      tiles_group(1, marched, mem, nt, off, lds);
     }
   }
   // Median, per (window, key width); small or F64 images run alone, and the
@@ -475,7 +483,10 @@ int launch_batch(ifm_ctx *ctx, const ifm_request *reqs, const int *idx, Block &b
                          tfirst);
       SHIP(hipGetLastError());
       break;
-    case 1: SHIP(launch_sep_batch((const SepReq *)(d + g.reqs), treq, tfirst, g.ntiles, g.lds, ctx->stream)); break;
+    case 1:
+      if (g.param) SHIP(launch_sep_march_batch((const SepReq *)(d + g.reqs), treq, tfirst, g.ntiles, ctx->stream));
+      else SHIP(launch_sep_batch((const SepReq *)(d + g.reqs), treq, tfirst, g.ntiles, g.lds, ctx->stream));
+      break;
     case 2:
       SHIP(launch_median_batch(g.param / 2, g.param % 2 == 1, (const MedianArgs *)(d + g.reqs), treq, tfirst,
                                g.ntiles, ctx->stream));

@@ -279,6 +279,101 @@ __global__ void __launch_bounds__(256) k_sep2d(Sep2dArgs a) {
   }
 }
 
+// Marching form (sep_march): wave g of the launch owns strip g % strips of
+// row chunk (g / strips) % chunks of plane g / (strips chunks); neighbouring
+// strips run on one XCD.
+struct SepMarchArgs {
+  Sep2dArgs s;
+  int strips, chunks, rows;  // rows per chunk
+  int64_t waves;
+};
+
+template <int K>
+__global__ void __launch_bounds__(256) k_sep_march(SepMarchArgs m) {
+  __shared__ __align__(16) float lds[4 * SM_R * sm_pitch(K)];
+  const Sep2dArgs &a = m.s;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t g = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * 4 + w;
+  if (g >= m.waves) return;  // the wave as a whole
+  const int strip = (int)(g % m.strips);
+  const int64_t t = g / m.strips;
+  const int chunk = (int)(t % m.chunks), plane = (int)(t / m.chunks);
+  const int p2 = plane % a.o2, p3 = plane / a.o2;
+  SepMarch q;
+  q.in = a.in;
+  q.out = a.out;
+  q.ibase = ((int64_t)(p2 + a.f2) + (int64_t)a.n2 * (p3 + a.f3)) * a.in_plane;
+  q.obase = (int64_t)plane * a.out_plane;
+  q.n0 = a.n0;
+  q.n1 = a.n1;
+  q.o0 = a.o0;
+  q.ox0 = strip * SM_W;
+  q.oy0 = chunk * m.rows;
+  q.nr = min(m.rows, a.o1 - q.oy0);
+  q.gx = a.f0 + q.ox0 + a.first0;
+  q.gy = a.f1 + q.oy0 + a.first1;
+  q.style = a.style;
+  q.dt_in = a.dt_in;
+  q.dt_out = a.dt_out;
+  q.fill = a.fill;
+  sep_march<K>(q, a.taps0, a.taps1, lds + w * SM_R * sm_pitch(K));
+}
+
+// Rows per chunk of a marched image: fewer rows make more waves, but every
+// chunk filters K - 1 rows beyond its own.  The chip is taken to be full with
+// `want` waves (four per SIMD while the registers allow, two above 17 taps).
+// 4096^2 F32: 13 taps 41 us with 32 rows (4096 waves), 46 with 64; 33 taps 93
+// and 82.
+constexpr int SM_MAXROWS = 64, SM_MINROWS = 16;  // sep_march stages at most 128 rows
+static int march_rows(int64_t o1, int64_t strips, int k) {
+  const double want = k <= 17 ? 4096 : 2048;
+  int best = SM_MAXROWS;
+  double cost = 0;
+  for (int rows = SM_MAXROWS; rows >= SM_MINROWS; rows /= 2) {
+    const double waves = (double)(strips * ((o1 + rows - 1) / rows));
+    const double c = (double)(rows + k - 1) / rows * std::max(1.0, want / waves);
+    if (rows == SM_MAXROWS || c < cost) {
+      best = rows;
+      cost = c;
+    }
+  }
+  return best;
+}
+
+// A wave marches for as long as the image has chunks of rows to spread over
+// the chip, so small images are faster in tiles: 1700 x 1200 F32, 9 / 13 / 33
+// taps: 11.9 / 13.5 / 22.8 us in tiles, 13.1 / 15.8 / 39.9 marched; 2500 x 1700:
+// 18.6 / 21.2 / 36.9 and 15.5 / 19.4 / 52.3; 4096^2 (5 / 13 / 33 taps): 58 / 66 /
+// 123 and 35 / 41 / 82.  The line is drawn at 4 M pixels, growing with the
+// taps beyond 13.
+constexpr int64_t SM_PIXELS = 4000000;
+
+bool sep_march_takes(int k0, int k1, int dt_in) {
+  const bool k = k0 == 3 || k0 == 5 || k0 == 7 || k0 == 9 || k0 == 13 || k0 == 17 || k0 == 21 || k0 == 25 || k0 == 29 ||
+                 k0 == 33;
+  return k0 == k1 && k && dt_in != IFM_F64;
+}
+
+static bool march_launch(const Sep2dArgs &s, hipStream_t st) {
+  if (!sep_march_takes(s.k0, s.k1, s.dt_in)) return false;
+  SepMarchArgs m;
+  m.s = s;
+  m.strips = (s.o0 + SM_W - 1) / SM_W;
+  m.rows = march_rows(s.o1, (int64_t)m.strips * s.nplanes, s.k0);
+  m.chunks = (s.o1 + m.rows - 1) / m.rows;
+  m.waves = (int64_t)m.strips * m.chunks * s.nplanes;
+  if ((int64_t)s.o0 * s.o1 * s.nplanes * 13 < SM_PIXELS * std::max(s.k0, 13) || m.waves > (int64_t(1) << 31))
+    return false;
+  const dim3 grid((unsigned)((m.waves + 3) / 4));
+  switch (s.k0) {
+#define MARCH(K) \
+  case K: hipLaunchKernelGGL(k_sep_march<K>, grid, dim3(256), 0, st, m); return true;
+    MARCH(3) MARCH(5) MARCH(7) MARCH(9) MARCH(13) MARCH(17) MARCH(21) MARCH(25) MARCH(29) MARCH(33)
+#undef MARCH
+  default: return false;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // sep3d: the three-factor cascade on axes 0, 1 and 2 in one pass.  A
 // workgroup owns a 64 x 32 column of outputs in (x, y) and up to S3_NZ output
@@ -536,6 +631,75 @@ __global__ void __launch_bounds__(256) k_sep_batch(const SepReq *__restrict__ re
   sep2d_tile(t, q.taps0, q.taps1, smem);
 }
 
+// The marched requests of a batch, of every length in one launch: workgroup g
+// runs waves 4 (g - tile_first[r]) .. + 3 of request r's strips and chunks.
+template <int K>
+__device__ __forceinline__ void march_req(const SepReq &q, const SepMarch &a, float *lds) {
+  // the taps into scalar registers: behind a pointer they would be read again
+  // after every store
+  float t0[K], t1[K];
+#pragma unroll
+  for (int t = 0; t < K; ++t) {
+    t0[t] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(q.taps0[t])));
+    t1[t] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(q.taps1[t])));
+  }
+  sep_march<K>(a, t0, t1, lds);
+}
+
+__global__ void __launch_bounds__(256) k_sep_march_batch(const SepReq *__restrict__ reqs,
+                                                         const int *__restrict__ tile_req,
+                                                         const int *__restrict__ tile_first) {
+  __shared__ __align__(16) float lds_all[4 * SM_R * sm_pitch(33)];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float *lds = lds_all + w * SM_R * sm_pitch(33);
+  const int g = xcd_tile(blockIdx.x, gridDim.x);
+  const int r = tile_req[g];
+  const SepReq &q = reqs[r];
+  const int unit = (g - tile_first[r]) * 4 + w, strips = (q.n0 + SM_W - 1) / SM_W;
+  SepMarch a;
+  a.in = q.in;
+  a.out = q.out;
+  a.ibase = a.obase = 0;
+  a.n0 = a.o0 = q.n0;
+  a.n1 = q.n1;
+  a.ox0 = (unit % strips) * SM_W;
+  a.oy0 = (unit / strips) * q.ty;
+  if (a.oy0 >= q.n1) return;  // the wave as a whole
+  a.nr = min(q.ty, q.n1 - a.oy0);
+  a.gx = a.ox0 + q.first0;
+  a.gy = a.oy0 + q.first1;
+  a.style = q.style;
+  a.dt_in = q.dt_in;
+  a.dt_out = q.dt_out;
+  a.fill = q.fill;
+  switch (q.k0) {
+  case 3: march_req<3>(q, a, lds); break;
+  case 5: march_req<5>(q, a, lds); break;
+  case 7: march_req<7>(q, a, lds); break;
+  case 9: march_req<9>(q, a, lds); break;
+  case 13: march_req<13>(q, a, lds); break;
+  case 17: march_req<17>(q, a, lds); break;
+  case 21: march_req<21>(q, a, lds); break;
+  case 25: march_req<25>(q, a, lds); break;
+  case 29: march_req<29>(q, a, lds); break;
+  default: march_req<33>(q, a, lds); break;
+  }
+}
+
+// Workgroups of a marched request, and its rows per chunk.
+int sep_march_groups(int n0, int n1, int *rows) {
+  *rows = 32;
+  const int64_t waves = (int64_t)((n0 + SM_W - 1) / SM_W) * ((n1 + *rows - 1) / *rows);
+  return (int)((waves + 3) / 4);
+}
+
+hipError_t launch_sep_march_batch(const SepReq *reqs, const int *tile_req, const int *tile_first, int ntiles,
+                                  hipStream_t st) {
+  if (ntiles == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_sep_march_batch, dim3(ntiles), dim3(256), 0, st, reqs, tile_req, tile_first);
+  return hipGetLastError();
+}
+
 hipError_t launch_sep_batch(const SepReq *reqs, const int *tile_req, const int *tile_first, int ntiles,
                             size_t lds_bytes, hipStream_t st) {
   if (ntiles == 0) return hipSuccess;
@@ -574,6 +738,7 @@ hipError_t launch_sep2d(const Dense4 &in, Dense4 &out, const int64_t *out_first,
   for (int t = 0; t < p1.len; ++t) a.taps1[t] = p1.taps[t];
   if (out.count() == 0) return hipSuccess;
   a.ty = ty;
+  if (march_launch(a, st)) return hipGetLastError();
   const size_t lds = sizeof(float) * sep2d_lds_floats(a.k0, a.k1, ty);
   dim3 grid((a.o0 + S2_TX - 1) / S2_TX, (a.o1 + ty - 1) / ty, a.nplanes < 65535 ? a.nplanes : 65535);
   hipLaunchKernelGGL(k_sep2d, grid, dim3(256), lds, st, a);

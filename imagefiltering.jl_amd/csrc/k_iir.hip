@@ -333,13 +333,6 @@ __device__ __forceinline__ Seg seg_lane(int n) {
   return g;
 }
 
-// LDS writes of this wave are seen by its own later reads.
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 struct State3 {
   double a, b, c;
 };

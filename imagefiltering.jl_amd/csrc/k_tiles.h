@@ -244,4 +244,190 @@ __device__ __forceinline__ void sep2d_tile(const Sep2dTile &a, const float *taps
   }
 }
 
+// ---------------------------------------------------------------------------
+// The same pair of factors for equal odd lengths K, by marching: a wave owns a
+// strip of 128 output columns (two per lane) and walks down the rows.  Each
+// staged row is filtered along axis 0 from the wave's own LDS row (two
+// outputs share K + 1 values read in pairs), and the result is added into the
+// K outputs of the column that still need it, kept in registers; the oldest
+// is complete and is stored.  The loads of the next SM_R rows are in flight
+// meanwhile.  Against the tile body above: no second LDS tile (5 LDS words
+// per output instead of 10 for K = 13), no rows staged twice within a strip,
+// constant tap counts, and no barrier.  Every sum runs in the same order
+// (taps ascending, from zero), so results are bit-identical.
+// ---------------------------------------------------------------------------
+constexpr int SM_W = 128;  // output columns of a strip
+constexpr int SM_R = 4;    // rows staged per step
+__host__ __device__ constexpr int sm_pitch(int k) { return SM_W + k - 1; }
+
+struct SepMarch {
+  const void *in;
+  void *out;
+  int64_t ibase, obase;  // plane offsets (elements)
+  int n0, n1, o0;        // input extents, output columns
+  int ox0, oy0, nr;      // output column and row of the strip's first output, its rows
+  int gx, gy;            // input column and row of the first staged element
+  int style, dt_in, dt_out;
+  float fill;
+};
+
+// How a strip's elements are loaded: FP32 pairs at any alignment (every staged
+// column is an image column), or one by one through the border map, by size.
+// One body per way, chosen once per wave: a choice per load would make the
+// loaded registers wait at its join.
+enum { SM_PAIRS = 0, SM_B32 = 1, SM_B16 = 2, SM_B8 = 3 };
+
+template <int LD>
+__device__ __forceinline__ void sm_issue(const SepMarch &a, const int (&sx)[4], bool halo, int64_t row, uint32_t (&v)[4]) {
+  if constexpr (LD == SM_PAIRS) {
+    const float *p = (const float *)a.in + row;
+    __builtin_memcpy(&v[0], p + sx[0], 8);
+    if (halo) __builtin_memcpy(&v[2], p + sx[2], 8);
+  } else {
+    using T = typename std::conditional<LD == SM_B32, uint32_t,
+              typename std::conditional<LD == SM_B16, uint16_t, uint8_t>::type>::type;
+    const T *p = (const T *)a.in + row;
+    v[0] = p[max(sx[0], 0)];
+    v[1] = p[max(sx[1], 0)];
+    if (halo) {
+      v[2] = p[max(sx[2], 0)];
+      v[3] = p[max(sx[3], 0)];
+    }
+  }
+}
+
+template <int LD>
+__device__ __forceinline__ float sm_val(const SepMarch &a, uint32_t r) {
+  if constexpr (LD == SM_B16) return a.dt_in == IFM_BF16 ? raw_val<IFM_BF16>(r) : raw_val<IFM_F16>(r);
+  else if constexpr (LD == SM_B8) return a.dt_in == IFM_N0F8 ? raw_val<IFM_N0F8>(r) : raw_val<IFM_U8>(r);
+  else return __uint_as_float(r);
+}
+
+template <int LD>
+__device__ __forceinline__ void sm_commit(const SepMarch &a, const int (&sx)[4], bool halo, bool fillrow,
+                                          const uint32_t (&v)[4], float *row) {
+  const int lane = threadIdx.x & 63;
+  float x[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x[i] = fillrow || (LD != SM_PAIRS && sx[i] < 0) ? a.fill : sm_val<LD>(a, v[i]);
+  *(float2 *)(row + 2 * lane) = make_float2(x[0], x[1]);
+  if (halo) *(float2 *)(row + SM_W + 2 * lane) = make_float2(x[2], x[3]);
+}
+
+// Two adjacent outputs of one row.
+__device__ __forceinline__ void sm_store(const SepMarch &a, int64_t o, bool two, float x, float y) {
+  switch (a.dt_out) {
+  case IFM_F32: {
+    float *p = (float *)a.out + o;
+    const float v[2] = {x, y};
+    if (two) __builtin_memcpy(p, v, 8);
+    else *p = x;
+    break;
+  }
+  case IFM_F64: {
+    double *p = (double *)a.out + o;
+    const double v[2] = {(double)x, (double)y};
+    if (two) __builtin_memcpy(p, v, 16);
+    else *p = v[0];
+    break;
+  }
+  default:
+    store_f(a.out, o, a.dt_out, x);
+    if (two) store_f(a.out, o + 1, a.dt_out, y);
+    break;
+  }
+}
+
+// lds: SM_R rows of sm_pitch(K) floats, the wave's own.  At most 128 staged
+// rows: lane l keeps the mapped image rows of staged rows l and l + 64.
+template <int K, int LD>
+__device__ __forceinline__ void sep_march_as(const SepMarch &a, const float *taps0, const float *taps1, float *lds) {
+  static_assert(K % 2 == 1 && K >= 3 && K <= 33, "odd, halo pairs on the wave's lanes");
+  constexpr int P = sm_pitch(K);
+  const int lane = threadIdx.x & 63;
+  const bool halo = lane < (K - 1) / 2;
+  int sx[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int x = a.gx + 2 * lane + (i & 1) + (i >> 1) * SM_W;
+    sx[i] = LD == SM_PAIRS ? x : bmap(a.style, x, a.n0);
+  }
+  const int nin = a.nr + K - 1;
+  const int sy0 = bmap(a.style, a.gy + min(lane, nin - 1), a.n1);
+  const int sy1 = bmap(a.style, a.gy + min(lane + 64, nin - 1), a.n1);
+  uint32_t v[SM_R][4];
+  uint32_t fillrows = 0;
+  auto issue = [&](int q0) {
+    fillrows = 0;
+#pragma unroll
+    for (int j = 0; j < SM_R; ++j) {
+      const int q = min(q0 + j, nin - 1);
+      const int sy = q < 64 ? __builtin_amdgcn_readlane(sy0, q) : __builtin_amdgcn_readlane(sy1, q - 64);
+      fillrows |= (sy < 0 ? 1u : 0u) << j;
+      sm_issue<LD>(a, sx, halo, a.ibase + (int64_t)max(sy, 0) * a.n0, v[j]);
+    }
+  };
+  auto commit = [&]() {
+#pragma unroll
+    for (int j = 0; j < SM_R; ++j) sm_commit<LD>(a, sx, halo, (fillrows >> j) & 1u, v[j], lds + j * P);
+  };
+  // A[c][i]: the output of column c that i + 1 more rows complete
+  float A[2][K - 1];
+#pragma unroll
+  for (int i = 0; i < K - 1; ++i) A[0][i] = A[1][i] = 0.f;
+  const int ox = a.ox0 + 2 * lane;
+  const bool two = ox + 1 < a.o0;
+  int64_t o = a.obase + (int64_t)a.oy0 * a.o0 + ox;
+  issue(0);
+#pragma unroll 1
+  for (int q0 = 0; q0 < nin; q0 += SM_R) {
+    commit();
+    wave_lds_fence();
+    if (q0 + SM_R < nin) issue(q0 + SM_R);
+#pragma unroll
+    for (int j = 0; j < SM_R; ++j) {
+      const float2 *src = (const float2 *)(lds + j * P) + lane;
+      float w[K + 1];
+#pragma unroll
+      for (int i = 0; i < (K + 1) / 2; ++i) {
+        const float2 t = src[i];
+        w[2 * i] = t.x;
+        w[2 * i + 1] = t.y;
+      }
+      float m0 = 0.f, m1 = 0.f;
+#pragma unroll
+      for (int t = 0; t < K; ++t) {
+        m0 = fmaf(taps0[t], w[t], m0);
+        m1 = fmaf(taps0[t], w[t + 1], m1);
+      }
+      const float r0 = fmaf(taps1[K - 1], m0, A[0][0]), r1 = fmaf(taps1[K - 1], m1, A[1][0]);
+#pragma unroll
+      for (int i = 0; i < K - 2; ++i) {
+        A[0][i] = fmaf(taps1[K - 2 - i], m0, A[0][i + 1]);
+        A[1][i] = fmaf(taps1[K - 2 - i], m1, A[1][i + 1]);
+      }
+      A[0][K - 2] = fmaf(taps1[0], m0, 0.f);
+      A[1][K - 2] = fmaf(taps1[0], m1, 0.f);
+      const int q = q0 + j;
+      if (q >= K - 1 && q < nin) {  // wave-uniform
+        if (ox < a.o0) sm_store(a, o, two, r0, r1);
+        o += a.o0;
+      }
+    }
+    wave_lds_fence();
+  }
+}
+
+template <int K>
+__device__ __forceinline__ void sep_march(const SepMarch &a, const float *taps0, const float *taps1, float *lds) {
+  if (a.dt_in == IFM_F32) {
+    if (a.gx >= 0 && a.gx + sm_pitch(K) <= a.n0) sep_march_as<K, SM_PAIRS>(a, taps0, taps1, lds);
+    else sep_march_as<K, SM_B32>(a, taps0, taps1, lds);
+  } else if (a.dt_in == IFM_BF16 || a.dt_in == IFM_F16) {
+    sep_march_as<K, SM_B16>(a, taps0, taps1, lds);
+  } else {
+    sep_march_as<K, SM_B8>(a, taps0, taps1, lds);
+  }
+}
+
 }  // namespace ifm

@@ -1201,3 +1201,36 @@ def test_median_float64_networks(k, shape):
                 want = O.median(xv.astype(np.float64), [-h, -h], [k, k], b)
                 got = IF.mapwindow(IF.median_, np.asfortranarray(x).view(IF.BF16Array), (k, k), border=b)
                 np.testing.assert_array_equal(IF.bf16_to_float32(got), want.astype(np.float32))
+
+
+# ---- marched pairs of factors ------------------------------------------------------------------
+@pytest.mark.parametrize("k", [3, 5, 7, 9, 13, 17, 21, 25, 29, 33])
+@pytest.mark.parametrize("shape", [(128, 35), (131, 70), (255, 17)])
+def test_fir_march_equals_tiles(k, shape):
+    """The marched form sums every output in the tiles' order: a stack of planes
+    large enough to be marched equals its planes filtered alone (too small to
+    be), bit for bit, over eltypes, borders, ragged strips and chunks, and an
+    output region that starts inside the image."""
+    rng = np.random.default_rng(k + shape[0])
+    taps = [rng.standard_normal(k), rng.standard_normal(k)]
+    planes = -(-4_000_000 * max(k, 13) // 13 // ((shape[0] - 2) * (shape[1] - 2))) + 1
+    vol = np.asfortranarray(rng.standard_normal(shape + (planes,)).astype(np.float32))
+    codes = np.asfortranarray(rng.integers(0, 256, shape + (planes,)).astype(np.uint8))
+    some = [0, planes // 2, planes - 1]
+    cases = [(vol, "reflect", IF.Float32), (vol, IF.Fill(0.5), IF.Float64), (codes, "circular", IF.Float32),
+             (IF.n0f8(codes), "symmetric", IF.Float64), (vol.astype(np.float16), "replicate", IF.Float32)]
+
+    def kern(n):
+        return tuple(IF.KernelFactors.ReshapedOneD(n, d, IF.centered(taps[d])) for d in range(2))
+
+    for a, b, T in cases:
+        got = np.asarray(IF.imfilter(T, a, kern(3), b, IF.Algorithm.FIRTiled()))
+        for z in some:
+            one = np.asfortranarray(a[:, :, z]).view(type(a))
+            np.testing.assert_array_equal(got[:, :, z], np.asarray(IF.imfilter(T, one, kern(2), b,
+                                                                               IF.Algorithm.FIRTiled())))
+    if min(shape) > k:
+        got = IF.imfilter(IF.Float32, vol, kern(3), IF.Inner(), IF.Algorithm.FIRTiled())
+        for z in some:
+            one = IF.imfilter(IF.Float32, np.asfortranarray(vol[:, :, z]), kern(2), IF.Inner(), IF.Algorithm.FIRTiled())
+            np.testing.assert_array_equal(np.asarray(got.data)[:, :, z], np.asarray(one.data))
