@@ -379,9 +379,9 @@ struct SepReq {
   float fill;
   int ty;  // tile height (S2_TY or S2_TY2), or rows per chunk of a marched request
 };
-// Whether a pair of factors can be marched (sep_march), and the workgroups and
-// rows per chunk of a marched request.
-bool sep_march_takes(int k0, int k1, int dt_in);
+// Whether a request is marched (sep_march) in a batch of so many pixels, and
+// the workgroups and rows per chunk of a marched request.
+bool sep_march_batched(int k0, int k1, int dt_in, int64_t batch_pixels);
 int sep_march_groups(int n0, int n1, int *rows);
 hipError_t launch_sep_march_batch(const SepReq *reqs, const int *tile_req, const int *tile_first, int ntiles,
                                   hipStream_t st);

@@ -272,8 +272,11 @@ int build_batch(ifm_ctx *ctx, const ifm_request *reqs, const int *idx, int n, co
     }
     if (!fr.empty()) tiles_group(0, 0, mem, nt, blk.put(fr.data(), fr.size() * sizeof(FillReq)), 0);
   }
-  // Separable: the marched requests and the ones in tiles.  A batch has rows
-  // enough to fill the chip by marching, whatever its images' sizes.
+  // Separable: the marched requests and the ones in tiles, by the pixels of the
+  // whole batch.
+  int64_t sep_pixels = 0;
+  for (int i = 0; i < n; ++i)
+    if (reqs[idx[i]].op == IFM_OP_SEPARABLE) sep_pixels += vin[i].n[0] * vin[i].n[1] * (reqs[idx[i]].nfactors2 > 0 ? 2 : 1);
   for (int marched = 0; marched < 2; ++marched) {
     std::vector<int> mem, nt;
     std::vector<SepReq> sr;
@@ -313,7 +316,7 @@ int build_batch(ifm_ctx *ctx, const ifm_request *reqs, const int *idx, int n, co
       s.dt_in = vin[i].dtype;
       s.dt_out = part ? q.out2.dtype : vout[i].dtype;
       s.fill = (float)q.border.fill;
-      if ((int)sep_march_takes(k0, k1, s.dt_in) != marched) continue;
+      if ((int)sep_march_batched(k0, k1, s.dt_in, sep_pixels) != marched) continue;
       int tiles;
       if (marched) {
         tiles = sep_march_groups(s.n0, s.n1, &s.ty);

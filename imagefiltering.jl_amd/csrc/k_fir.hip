@@ -346,9 +346,9 @@ static int march_rows(int64_t o1, int64_t strips, int k) {
 // 18.6 / 21.2 / 36.9 and 15.5 / 19.4 / 52.3; 4096^2 (5 / 13 / 33 taps): 58 / 66 /
 // 123 and 35 / 41 / 82.  The line is drawn at 4 M pixels, growing with the
 // taps beyond 13.
-constexpr int64_t SM_PIXELS = 4000000;
+constexpr int64_t SM_PIXELS = 4000000, SM_BATCH_PIXELS = 16000000;
 
-bool sep_march_takes(int k0, int k1, int dt_in) {
+static bool sep_march_takes(int k0, int k1, int dt_in) {
   const bool k = k0 == 3 || k0 == 5 || k0 == 7 || k0 == 9 || k0 == 13 || k0 == 17 || k0 == 21 || k0 == 25 || k0 == 29 ||
                  k0 == 33;
   return k0 == k1 && k && dt_in != IFM_F64;
@@ -684,6 +684,15 @@ __global__ void __launch_bounds__(256) k_sep_march_batch(const SepReq *__restric
   case 29: march_req<29>(q, a, lds); break;
   default: march_req<33>(q, a, lds); break;
   }
+}
+
+// In a batch the marched requests share one kernel (the registers of the
+// longest factors) and end with its longest waves, so the line is drawn higher
+// than for one image.  Batches of the serving mix (sides up to 2048), in tiles
+// and marched: 24 requests 143 / 172 us, 48: 231 / 246, 96: 441 / 393, 256: 830
+// / 715.
+bool sep_march_batched(int k0, int k1, int dt_in, int64_t batch_pixels) {
+  return sep_march_takes(k0, k1, dt_in) && batch_pixels * 13 >= SM_BATCH_PIXELS * std::max(k0, 13);
 }
 
 // Workgroups of a marched request, and its rows per chunk.
