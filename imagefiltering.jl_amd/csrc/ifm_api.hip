@@ -247,8 +247,8 @@ int sep2d_tile_h(const ifm_ctx *ctx, int dt_in, int k0, int k1, int64_t pixels) 
 }  // namespace ifm
 
 // all(isfinite, a) for filter_algorithm (src/imfilter.jl:1200-1209): one
-// streaming read, a flag set by any lane that meets an Inf or NaN.
-__global__ void __launch_bounds__(256) k_all_finite(const void *p, int64_t count, int dt, int vec, int *flag) {
+// streaming read, a flag set to gen by any lane that meets an Inf or NaN.
+__global__ void __launch_bounds__(256) k_all_finite(const void *p, int64_t count, int dt, int vec, int *flag, int gen) {
   const int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   bool bad = false;
@@ -272,7 +272,15 @@ __global__ void __launch_bounds__(256) k_all_finite(const void *p, int64_t count
     const uint32_t m = dt == IFM_BF16 ? 0x7f80u : 0x7c00u;
     for (int64_t i = tid; i < count; i += stride) bad |= (((const uint16_t *)p)[i] & m) == m;
   }
-  if (bad) atomicOr(flag, 1);
+  if (bad) atomicExch(flag, gen);
+}
+
+static hipError_t launch_all_finite(const void *p, int64_t count, int dt, int *flag, int gen, hipStream_t st) {
+  const bool vec = dt == IFM_F32 && ((uintptr_t)p & 15) == 0;
+  const int64_t units = vec ? (count + 3) / 4 : count;
+  const int64_t blocks = std::min<int64_t>((units + 255) / 256, 4096);
+  hipLaunchKernelGGL(k_all_finite, dim3((unsigned)blocks), dim3(256), 0, st, p, count, dt, vec ? 1 : 0, flag, gen);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -321,12 +329,7 @@ int ifm_all_finite(ifm_ctx *ctx, const ifm_array *a, int *result) {
     return fail(ctx, IFM_E_NOMEM, "device allocation failed (finite flag)");
   }
   HIPCHK(hipMemsetAsync(ctx->finite_flag, 0, sizeof(int), ctx->stream));
-  const bool vec = dt == IFM_F32 && ((uintptr_t)a->data & 15) == 0;
-  const int64_t units = vec ? (count + 3) / 4 : count;
-  const int64_t blocks = std::min<int64_t>((units + 255) / 256, 4096);
-  hipLaunchKernelGGL(k_all_finite, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, a->data, count, dt,
-                     vec ? 1 : 0, ctx->finite_flag);
-  HIPCHK(hipGetLastError());
+  HIPCHK(launch_all_finite(a->data, count, dt, ctx->finite_flag, 1, ctx->stream));
   int h = 0;
   HIPCHK(hipMemcpyAsync(&h, ctx->finite_flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -485,7 +488,6 @@ int ifm_ctx_destroy(ifm_ctx *ctx) {
     (void)hipFree(e.tw64);
   }
   for (auto &e : ctx->tile_spec) (void)hipFree(e.spec);
-  if (ctx->tile_taps) (void)hipFree(ctx->tile_taps);
   if (ctx->tile_flag) (void)hipFree(ctx->tile_flag);
   if (ctx->finite_flag) (void)hipFree(ctx->finite_flag);
   batch_release(ctx);
@@ -930,11 +932,13 @@ static int tile_twiddles(ifm_ctx *ctx, int F, const float2 **tw32, const double2
 }
 
 // The kernel's F x F spectrum for the tiled FFT, cached per ctx and keyed by
-// the exact FP32 taps, the kernel shape and F.
-static int tile_spectrum(ifm_ctx *ctx, const DenseKernel &dk, int F, const double2 *tw64, const float2 **spec) {
+// the exact FP32 taps, the kernel shape and F.  The entry also holds the taps
+// on the device and room for their Toeplitz table (ifm_imfilter_default).
+static int tile_spectrum(ifm_ctx *ctx, const DenseKernel &dk, int F, const double2 *tw64,
+                         const ifm_ctx::TileSpec **spec) {
   for (auto &e : ctx->tile_spec)
     if (e.F == F && e.k0 == dk.n[0] && e.k1 == dk.n[1] && e.taps == dk.taps) {
-      *spec = (const float2 *)e.spec;
+      *spec = &e;
       return IFM_OK;
     }
   if (ctx->tile_spec.size() >= 16) {  // bounded cache: drop the oldest entry
@@ -943,28 +947,100 @@ static int tile_spectrum(ifm_ctx *ctx, const DenseKernel &dk, int F, const doubl
     ctx->tile_spec.erase(ctx->tile_spec.begin());
   }
   const size_t tb = dk.taps.size() * sizeof(float);
-  if (ctx->tile_taps_bytes < tb) {
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (ctx->tile_taps) HIPCHK(hipFree(ctx->tile_taps));
-    ctx->tile_taps = nullptr;
-    ctx->tile_taps_bytes = 0;
-    if (hipMalloc(&ctx->tile_taps, tb) != hipSuccess) return fail(ctx, IFM_E_NOMEM, "device allocation failed (FFT taps)");
-    ctx->tile_taps_bytes = tb;
-  }
+  ToeplitzJob job;
+  float kinv;
+  const auto up = [](size_t x) { return (x + 255) / 256 * 256; };
   ifm_ctx::TileSpec e;
   e.F = F;
   e.k0 = dk.n[0];
   e.k1 = dk.n[1];
   e.taps = dk.taps;
-  if (hipMalloc(&e.spec, fft_tile_spec_bytes(F)) != hipSuccess)
+  e.taps_off = up(fft_tile_spec_bytes(F));
+  e.table_off = e.taps_off + up(tb);
+  const size_t table = dk.n[0] <= 49 && dk.n[1] <= 32 ? dense_mfma_job(dk, &job, &kinv) : 0;
+  if (hipMalloc(&e.spec, e.table_off + table) != hipSuccess)
     return fail(ctx, IFM_E_NOMEM, "device allocation failed (FFT kernel spectrum)");
   ctx->tile_spec.push_back(std::move(e));
   ifm_ctx::TileSpec &h = ctx->tile_spec.back();
+  float *d_taps = (float *)((char *)h.spec + h.taps_off);
   // the entry keeps the host taps alive until it is dropped (after a stream sync)
-  HIPCHK(hipMemcpyAsync(ctx->tile_taps, h.taps.data(), tb, hipMemcpyHostToDevice, ctx->stream));
-  HIPCHK(launch_fft_tile_spectrum((const float *)ctx->tile_taps, dk.n[0], dk.n[1], F, tw64, (float2 *)h.spec,
-                                  ctx->stream));
-  *spec = (const float2 *)h.spec;
+  HIPCHK(hipMemcpyAsync(d_taps, h.taps.data(), tb, hipMemcpyHostToDevice, ctx->stream));
+  HIPCHK(launch_fft_tile_spectrum(d_taps, dk.n[0], dk.n[1], F, tw64, (float2 *)h.spec, ctx->stream));
+  *spec = &h;
+  return IFM_OK;
+}
+
+// The tiled transform of one call: its tables, the kernel's cache entry, the
+// non-finite flag and this call's generation of it.
+static int tile_setup(ifm_ctx *ctx, const DenseKernel &dk, int F, const float2 **tw32,
+                      const ifm_ctx::TileSpec **spec) {
+  const double2 *tw64;
+  int rc;
+  if ((rc = tile_twiddles(ctx, F, tw32, &tw64))) return rc;
+  if ((rc = tile_spectrum(ctx, dk, F, tw64, spec))) return rc;
+  if (!ctx->tile_flag) {
+    if (hipMalloc(&ctx->tile_flag, sizeof(int)) != hipSuccess)
+      return fail(ctx, IFM_E_NOMEM, "device allocation failed (FFT flag)");
+    HIPCHK(hipMemsetAsync(ctx->tile_flag, 0, sizeof(int), ctx->stream));
+  }
+  if (++ctx->tile_gen <= 0) ctx->tile_gen = 1;
+  return IFM_OK;
+}
+
+// The scan costs one read of the image (5 us at 3000 x 2001 F32) and the two
+// launches that find nothing to do about 4 us; waiting for the scan's answer
+// on the host cost 45 us of each call (3000 x 2001, 21 x 21: 109 us a call,
+// the transform itself 55).
+int ifm_imfilter_default(ifm_ctx *ctx, const ifm_array *in, ifm_array *out, const ifm_kernel *kernel,
+                         const ifm_border *b) {
+  if (!ctx) return IFM_E_ARG;
+  Geo g;
+  int rc;
+  if ((rc = common_setup(ctx, in, out, g))) return rc;
+  if ((rc = check_border(ctx, b))) return rc;
+  if (!is_float_out(out->dtype)) return fail(ctx, IFM_E_UNSUPPORTED, "imfilter: output eltype must be floating point");
+  DenseKernel dk;
+  if ((rc = dense_kernel_canon(ctx, kernel, g, in->ndim, dk))) return rc;
+  const int F = fft_tile_size(dk);
+  bool ok = in->device && out->device && is_float_out(in->dtype) && F > 0 && dk.n[0] <= 64 && dk.n[1] <= 64 &&
+            (b->style != IFM_FILL || isfinite((float)b->fill));
+  for (int d = 0; d < in->ndim; ++d) ok = ok && in->size[d] == out->size[d];
+  // every pixel lies in its own output's window, so the scan and the
+  // transform see the same pixels
+  for (int m = 0; m < 2; ++m) ok = ok && dk.first[m] <= 0 && dk.first[m] + dk.n[m] > 0;
+  if (!ok) return fail(ctx, IFM_E_UNSUPPORTED, "ifm_imfilter_default: not a tiled 2-D transform of a device array");
+  View vi, vo;
+  if ((rc = make_view(ctx, in, g, S_IN, true, vi))) return rc;
+  if ((rc = make_view(ctx, out, g, S_OUT, false, vo))) return rc;
+  bool padded[MAXD];
+  for (int m = 0; m < MAXD; ++m) padded[m] = dk.n[m] > 1 || dk.first[m] != 0;
+  if ((rc = check_reflect(ctx, b, vi.d, padded))) return rc;
+  if (vo.d.count() == 0) return IFM_OK;
+  const float2 *tw32;
+  const ifm_ctx::TileSpec *spec;
+  if ((rc = tile_setup(ctx, dk, F, &tw32, &spec))) return rc;
+  const int64_t of[MAXD] = {0, 0, 0, 0};
+  const float fill = (float)b->fill;
+  const float *d_taps = (const float *)((const char *)spec->spec + spec->taps_off);
+  HIPCHK(launch_all_finite(vi.d.data, vi.d.count(), vi.d.dtype, ctx->tile_flag, ctx->tile_gen, ctx->stream));
+  HIPCHK(launch_fft_tile(vi.d, vo.d, of, dk, F, (const float2 *)spec->spec, tw32, ctx->tile_flag, ctx->tile_gen,
+                         b->style, fill, true, ctx->stream));
+  // the direct sum, where the scan met an Inf or NaN, as ifm_imfilter_dense
+  // would take it
+  Gate gate;
+  gate.flag = ctx->tile_flag;
+  gate.gen = ctx->tile_gen;
+  if (dk.n[0] >= 15 && dk.n[1] >= 15 && dense_mfma_supported(dk, vi.d, vo.d)) {
+    ToeplitzJob job;
+    float kinv;
+    dense_mfma_job(dk, &job, &kinv);
+    job.taps = d_taps;
+    job.table = (uint16_t *)((char *)spec->spec + spec->table_off);
+    HIPCHK(launch_toeplitz_one(job, gate, ctx->stream));
+    HIPCHK(launch_dense_mfma(vi.d, vo.d, of, dk, job.table, d_taps, kinv, b->style, fill, ctx->stream, gate));
+  } else {
+    HIPCHK(launch_dense_valu(vi.d, vo.d, of, dk, d_taps, b->style, fill, ctx->stream, gate));
+  }
   return IFM_OK;
 }
 
@@ -993,18 +1069,10 @@ int ifm_imfilter_fft(ifm_ctx *ctx, const ifm_array *in, ifm_array *out, const in
   if (F > 0) {
     if (vo.d.count() > 0) {
       const float2 *tw32;
-      const double2 *tw64;
-      const float2 *spec;
-      if ((rc = tile_twiddles(ctx, F, &tw32, &tw64))) return rc;
-      if ((rc = tile_spectrum(ctx, dk, F, tw64, &spec))) return rc;
-      if (!ctx->tile_flag) {
-        if (hipMalloc(&ctx->tile_flag, sizeof(int)) != hipSuccess)
-          return fail(ctx, IFM_E_NOMEM, "device allocation failed (FFT flag)");
-        HIPCHK(hipMemsetAsync(ctx->tile_flag, 0, sizeof(int), ctx->stream));
-      }
-      if (++ctx->tile_gen <= 0) ctx->tile_gen = 1;
-      HIPCHK(launch_fft_tile(vi.d, vo.d, of, dk, F, spec, tw32, ctx->tile_flag, ctx->tile_gen, b->style,
-                             (float)b->fill, ctx->stream));
+      const ifm_ctx::TileSpec *spec;
+      if ((rc = tile_setup(ctx, dk, F, &tw32, &spec))) return rc;
+      HIPCHK(launch_fft_tile(vi.d, vo.d, of, dk, F, (const float2 *)spec->spec, tw32, ctx->tile_flag, ctx->tile_gen,
+                             b->style, (float)b->fill, false, ctx->stream));
     }
     if ((rc = finish_view(ctx, vo))) return rc;
     return sync_if_host(ctx, !in->device || !out->device);

@@ -224,6 +224,14 @@ bool sep3d_supported(int k0, int k1, int k2, int dt_in, int64_t plane_elems);
 hipError_t launch_sep3d(const Dense4 &in, Dense4 &out, const int64_t *out_first, const FirPass &p0, const FirPass &p1,
                         const FirPass &p2, int style, float fill, hipStream_t st);
 
+// A launch that does its work only where an earlier kernel of the stream set
+// *flag to gen (flag NULL: always).
+struct Gate {
+  const int *flag = nullptr;
+  int gen = 0;
+};
+__device__ __forceinline__ bool gate_closed(const Gate &g) { return g.flag && *g.flag != g.gen; }
+
 struct DenseKernel {
   int ndim;
   int n[MAXD];
@@ -231,7 +239,7 @@ struct DenseKernel {
   std::vector<float> taps;  // column-major
 };
 hipError_t launch_dense_valu(const Dense4 &in, Dense4 &out, const int64_t *out_first, const DenseKernel &k,
-                             const float *d_taps, int style, float fill, hipStream_t st);
+                             const float *d_taps, int style, float fill, hipStream_t st, Gate gate = Gate());
 // Matrix-core banded-Toeplitz path (2-D kernels up to 49 x 32).
 struct MfmaArgs {
   const void *in;
@@ -250,6 +258,7 @@ struct MfmaArgs {
   int style;
   int dt_in, dt_out;
   float fill;
+  Gate gate;
 };
 bool dense_mfma_supported(const DenseKernel &k, const Dense4 &in, const Dense4 &out);
 void dense_mfma_table(const DenseKernel &k, std::vector<uint16_t> &table, float *kinv);
@@ -267,9 +276,10 @@ struct ToeplitzJob {
 };
 size_t dense_mfma_job(const DenseKernel &k, ToeplitzJob *job, float *kinv);  // returns the table bytes
 hipError_t launch_toeplitz(const ToeplitzJob *jobs, int njobs, hipStream_t st);
+hipError_t launch_toeplitz_one(const ToeplitzJob &job, Gate gate, hipStream_t st);
 hipError_t launch_dense_mfma(const Dense4 &in, Dense4 &out, const int64_t *out_first, const DenseKernel &k,
                              const uint16_t *d_table, const float *d_taps, float kinv, int style, float fill,
-                             hipStream_t st);
+                             hipStream_t st, Gate gate = Gate());
 hipError_t launch_dense_mfma_batch(int variant, const MfmaArgs *reqs, const int *tile_req, const int *tile_first,
                                    int ntiles, hipStream_t st);
 
@@ -346,11 +356,13 @@ size_t fft_tile_spec_bytes(int F);
 void fft_tile_twiddles(int F, std::vector<float2> &tw32, std::vector<double2> &tw64);
 hipError_t launch_fft_tile_spectrum(const float *d_taps, int K0, int K1, int F, const double2 *tw64, float2 *spec,
                                     hipStream_t st);
-// nanflag / gen: a non-finite input value (or Fill value) sets *nanflag = gen
+// skip: the launch does nothing where *nanflag is already gen, and the output
+// is then left to the caller; a non-finite Fill value must not be given.
+// Otherwise, nanflag / gen: a non-finite input value (or Fill value) sets *nanflag = gen
 // and the whole output becomes NaN, as the whole-array transform gives.
 hipError_t launch_fft_tile(const Dense4 &in, Dense4 &out, const int64_t *out_first, const DenseKernel &k, int F,
                            const float2 *spec, const float2 *tw32, int *nanflag, int gen, int style, float fill,
-                           hipStream_t st);
+                           bool skip, hipStream_t st);
 
 // Elementwise passes (k_elem.hip): NaN mask and zero-filled copy (hasna set
 // when a NaN is met), num /= den, and a dense src copied into dst at dst_first.
@@ -447,11 +459,10 @@ struct ifm_ctx {
   struct TileSpec {
     int F = 0, k0 = 0, k1 = 0;
     std::vector<float> taps;
-    void *spec = nullptr;
+    void *spec = nullptr;   // the spectrum, the FP32 taps, and room for their Toeplitz table
+    size_t taps_off = 0, table_off = 0;
   };
   std::vector<TileSpec> tile_spec;
-  void *tile_taps = nullptr;  // device staging of the taps being transformed
-  size_t tile_taps_bytes = 0;
   int *tile_flag = nullptr;   // non-finite flag of the tile kernel
   int tile_gen = 0;
   // device address of the no-alloc scratch array on this ctx's device

@@ -83,10 +83,12 @@ struct Dense2dArgs {
   int style;
   int dt_in, dt_out;
   float fill;
+  Gate gate;
 };
 
 __global__ void __launch_bounds__(256) k_dense2d_valu(Dense2dArgs a) {
   extern __shared__ float smem[];
+  if (gate_closed(a.gate)) return;
   const int IN_W = DV_TX + a.k0 - 1;
   const int IN_H = DV_TY + a.k1 - 1;
   const int IN_WP = IN_W | 1;
@@ -161,6 +163,7 @@ __global__ void __launch_bounds__(256) k_dense2d_small(Dense2dArgs a, SmallTaps<
   constexpr int NE = IN_H * IN_W, NI = (NE + 255) / 256;
   __shared__ float smem[IN_H * IN_WP];
   __shared__ int smap[IN_H + IN_W];  // border tiles: source row of tile row r, then source column of tile column c
+  if (gate_closed(a.gate)) return;
   const int tid = threadIdx.x;
   const int tx = tid & 63, ty = tid >> 6;
   const int tile = xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
@@ -473,7 +476,7 @@ static hipError_t launch_dense3d(const Dense4 &in, Dense4 &out, const int64_t *o
 }
 
 hipError_t launch_dense_valu(const Dense4 &in, Dense4 &out, const int64_t *out_first, const DenseKernel &k,
-                             const float *d_taps, int style, float fill, hipStream_t st) {
+                             const float *d_taps, int style, float fill, hipStream_t st, Gate gate) {
   if (out.count() == 0) return hipSuccess;
   bool twod = k.ndim <= 2 || (k.n[2] == 1 && k.n[3] == 1);
   if (twod && k.n[0] <= 64 && k.n[1] <= 64) {
@@ -502,6 +505,7 @@ hipError_t launch_dense_valu(const Dense4 &in, Dense4 &out, const int64_t *out_f
     a.dt_in = in.dtype;
     a.dt_out = out.dtype;
     a.fill = fill;
+    a.gate = gate;
     const int IN_W = DV_TX + a.k0 - 1, IN_H = DV_TY + a.k1 - 1;
     size_t lds = sizeof(float) * (size_t)IN_H * (IN_W | 1);
     dim3 grid((a.o0 + DV_TX - 1) / DV_TX, (a.o1 + DV_TY - 1) / DV_TY, a.nplanes < 65535 ? a.nplanes : 65535);
@@ -521,6 +525,7 @@ hipError_t launch_dense_valu(const Dense4 &in, Dense4 &out, const int64_t *out_f
     hipLaunchKernelGGL(k_dense2d_valu, grid, dim3(256), lds, st, a);
     return hipGetLastError();
   }
+  if (gate.flag) return hipErrorInvalidValue;  // 2-D kernels of up to 64 taps per axis only
   const bool threed = k.ndim >= 3 && (k.ndim < 4 || k.n[3] == 1) && small3_size(k.n[0]) && small3_size(k.n[1]) &&
                       small3_size(k.n[2]);
   if (threed && (out.n[2] + D3_NZ - 1) / D3_NZ * out.n[3] <= 65535)

@@ -122,6 +122,7 @@ struct FftTileArgs {
   int o2, n2, of2, of3; // plane mapping of axes 2 and 3
   int style, dt_in, dt_out;
   float fill;
+  int skip;             // nothing to do where *nanflag is gen already
 };
 
 template <int F>
@@ -150,6 +151,7 @@ __global__ void __launch_bounds__(TileCfg<F>::NT) k_fft_tile(FftTileArgs a) {
   static_assert(T1N * R1 == V && T2N * R2 == V, "task split");
   static_assert(NT % F == 0 || F % 64 == 0, "line-fastest lanes");
   extern __shared__ float2 lds[];
+  if (a.skip && *a.nanflag == a.gen) return;
   const int t = threadIdx.x;
   float2 v[V];
 
@@ -409,7 +411,7 @@ hipError_t launch_fft_tile_spectrum(const float *d_taps, int K0, int K1, int F, 
 
 hipError_t launch_fft_tile(const Dense4 &in, Dense4 &out, const int64_t *out_first, const DenseKernel &k, int F,
                            const float2 *spec, const float2 *tw32, int *nanflag, int gen, int style, float fill,
-                           hipStream_t st) {
+                           bool skip, hipStream_t st) {
   FftTileArgs a;
   a.in = in.data;
   a.out = out.data;
@@ -441,6 +443,7 @@ hipError_t launch_fft_tile(const Dense4 &in, Dense4 &out, const int64_t *out_fir
   a.dt_in = in.dtype;
   a.dt_out = out.dtype;
   a.fill = fill;
+  a.skip = skip;
   if (a.ntiles == 0) return hipSuccess;
   const int64_t pairs = (a.ntiles + 1) / 2;
   if (pairs > 0x7fffffff) return hipErrorInvalidValue;
@@ -450,7 +453,7 @@ hipError_t launch_fft_tile(const Dense4 &in, Dense4 &out, const int64_t *out_fir
     hipLaunchKernelGGL(k_fft_tile<128>, dim3((unsigned)pairs), dim3(TileCfg<128>::NT), tile_lds_bytes<128>(), st,
                        a);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess || skip) return e;
   const int64_t total = out.count();
   const int64_t blocks = std::min<int64_t>((total + 255) / 256, 1024);
   hipLaunchKernelGGL(k_fft_nanfill, dim3((unsigned)blocks), dim3(256), 0, st, out.data, out.n[0] * out.n[1], nplanes,

@@ -552,6 +552,7 @@ __global__ void __launch_bounds__(256, 2) k_dense_mfma(MfmaArgs a0, MfBatch bt) 
   extern __shared__ __attribute__((aligned(16))) uint32_t lds32[];
   __shared__ float red[2][MF_WAVES];
   __shared__ int redflag[2][MF_WAVES];
+  if (gate_closed(a0.gate)) return;
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 15, lgrp = lane >> 4;
@@ -815,6 +816,21 @@ size_t dense_mfma_job(const DenseKernel &k, ToeplitzJob *job, float *kinv) {
   return (size_t)job->kb * job->urows * 64 * 8 * 2 * sizeof(uint16_t);
 }
 
+// One table, a workgroup per 256 entries.
+__global__ void __launch_bounds__(256) k_toeplitz_one(ToeplitzJob j, Gate gate) {
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (gate_closed(gate) || e >= j.kb * j.urows * 64 * 8) return;
+  uint16_t h, l;
+  const size_t pos = toeplitz_entry(j.taps, j.kx, j.ky, j.urows, j.ks, e, &h, &l);
+  j.table[pos] = h;
+  j.table[pos + 64 * 8] = l;
+}
+
+hipError_t launch_toeplitz_one(const ToeplitzJob &job, Gate gate, hipStream_t st) {
+  hipLaunchKernelGGL(k_toeplitz_one, dim3((job.kb * job.urows * 64 * 8 + 255) / 256), dim3(256), 0, st, job, gate);
+  return hipGetLastError();
+}
+
 hipError_t launch_toeplitz(const ToeplitzJob *jobs, int njobs, hipStream_t st) {
   if (njobs == 0) return hipSuccess;
   hipLaunchKernelGGL(k_toeplitz, dim3(njobs), dim3(256), 0, st, jobs);
@@ -853,6 +869,7 @@ bool dense_mfma_args(const Dense4 &in, Dense4 &out, const int64_t *out_first, co
   a.dt_in = in.dtype;
   a.dt_out = out.dtype;
   a.fill = fill;
+  a.gate = Gate();
   a.ntx = (a.o0 + MF_TX - 1) / MF_TX;
   a.nty = (a.o1 + MF_TY - 1) / MF_TY;
   const int64_t ntiles = (int64_t)a.ntx * a.nty * out.n[2] * out.n[3];
@@ -869,13 +886,14 @@ static int64_t mf_grid(int64_t ntiles) {
 
 hipError_t launch_dense_mfma(const Dense4 &in, Dense4 &out, const int64_t *out_first, const DenseKernel &k,
                              const uint16_t *d_table, const float *d_taps, float kinv, int style, float fill,
-                             hipStream_t st) {
+                             hipStream_t st, Gate gate) {
   if (out.count() == 0) return hipSuccess;
   MfVariant v;
   MfmaArgs a;
   if (!mf_select(mfma_kb(k.n[0]), mfma_nch(k.n[1]), &v) ||
       !dense_mfma_args(in, out, out_first, k, d_table, d_taps, kinv, style, fill, &a))
     return hipErrorInvalidValue;
+  a.gate = gate;
   // a 15-row kernel in one K block sweeps 15 rows, not the padded 16
   if (mfma_kb(k.n[0]) == 1 && k.n[1] == 15) v = mf_variant<1, 2, 15>();
   MfBatch none = {nullptr, nullptr, nullptr};

@@ -82,7 +82,7 @@ MAX_TILE_RULES = 256
 EXPORTS = [
     "ifm_ctx_create", "ifm_ctx_destroy", "ifm_ctx_set_stream", "ifm_ctx_synchronize", "ifm_last_error",
     "ifm_version", "ifm_padarray", "ifm_imfilter_fir", "ifm_imfilter_fir_noalloc", "ifm_imfilter_dense", "ifm_all_finite", "ifm_na_prepare", "ifm_divide",
-    "ifm_copy_into", "ifm_local_extrema", "ifm_convert_int", "ifm_imfilter_fft",
+    "ifm_copy_into", "ifm_local_extrema", "ifm_convert_int", "ifm_imfilter_fft", "ifm_imfilter_default",
     "ifm_imfilter_iir", "ifm_mapwindow_median", "ifm_mapwindow_minmax", "ifm_extrema_filter", "ifm_mapwindow_generic",
     "ifm_batch_run", "ifm_serve", "ifm_fill_uniform",
     "ifm_server_create", "ifm_server_submit", "ifm_server_poll", "ifm_server_wait", "ifm_server_destroy",
@@ -120,6 +120,7 @@ def load(path=LIBPATH):
     L.ifm_imfilter_dense.argtypes = [vp, P(IfmArray), P(IfmArray), P(C.c_int64), P(IfmKernel), P(IfmBorder),
                                      C.c_int]
     L.ifm_imfilter_fft.argtypes = [vp, P(IfmArray), P(IfmArray), P(C.c_int64), P(IfmKernel), P(IfmBorder)]
+    L.ifm_imfilter_default.argtypes = [vp, P(IfmArray), P(IfmArray), P(IfmKernel), P(IfmBorder)]
     L.ifm_all_finite.argtypes = [vp, P(IfmArray), P(C.c_int)]
     L.ifm_na_prepare.argtypes = [vp, P(IfmArray), P(IfmArray), P(IfmArray), P(C.c_int)]
     L.ifm_divide.argtypes = [vp, P(IfmArray), P(IfmArray)]

@@ -554,6 +554,8 @@ def imfilter(*args):
     if isinstance(border, (Pad, Fill)):
         _check_explicit_padding(border, kernel, N)
     out = empty_like(img, T)
+    if r is None and alg is None and _run_default(out, img, kernel, border):
+        return out
     return _run(_choose(r, alg, img, kernel), out, img, kernel, border, None)
 
 
@@ -575,6 +577,24 @@ def _choose(r, alg, img, kernel):
     if alg is None:
         alg = filter_algorithm(img, kernel)
     return alg
+
+
+def _run_default(out, img, kernel, border):
+    """filter_algorithm's choice for one long dense kernel on a device array,
+    made on the device (ifm_imfilter_default); False where the host decides."""
+    if not (len(kernel) == 1 and isinstance(kernel[0], OffsetArray) and isinstance(border, (Pad, Fill))
+            and isinstance(img, DeviceArray) and img.eltype.kind == "float" and maxlen(kernel) > 30):
+        return False
+    comps = _components(kernel, len(img.shape))
+    if len(comps) != 1 or comps[0].kind != "dense":
+        return False
+    kk = _kernel_struct(_comp_dense(comps[0], len(img.shape)))
+    rc = _lib.load().ifm_imfilter_default(_lib.ctx(), ifm_array(img), ifm_array(out), kk,
+                                          _border_struct(border, img.eltype))
+    if rc == _lib.E_UNSUPPORTED:
+        return False
+    _lib.check(rc)
+    return True
 
 
 def imfilter_(*args):

@@ -1234,3 +1234,38 @@ def test_fir_march_equals_tiles(k, shape):
         for z in some:
             one = IF.imfilter(IF.Float32, np.asfortranarray(vol[:, :, z]), kern(2), IF.Inner(), IF.Algorithm.FIRTiled())
             np.testing.assert_array_equal(np.asarray(got.data)[:, :, z], np.asarray(one.data))
+
+
+# ---- the default algorithm of one long dense kernel, chosen on the device ----------------------
+@pytest.mark.parametrize("kshape", [(7, 7), (8, 6), (15, 15), (21, 17), (31, 31), (33, 20), (45, 45)])
+def test_default_algorithm_on_device(kshape):
+    """imfilter(img, kernel, border) on device arrays equals the algorithm that
+    filter_algorithm names, bit for bit: FFT for finite images, FIR for images
+    with an Inf or NaN anywhere (first and last pixel, inside), the kernels the
+    device does not take included (a non-finite Fill, a window off its origin)."""
+    rng = np.random.default_rng(kshape[0])
+    taps = rng.standard_normal(kshape)
+    kern = IF.centered(taps)
+    off = IF.OffsetArray(taps, (2, -1))
+    img = rng.random((150, 133)).astype(np.float32)
+    images = [img]
+    for at, v in (((0, 0), np.nan), ((149, 132), np.inf), ((70, 3), -np.inf)):
+        x = img.copy()
+        x[at] = v
+        images.append(x)
+    images.append(np.asfortranarray(images[1]))
+    images.append(images[3].astype(np.float64))
+    for n, x in enumerate(images):
+        d = IF.DeviceArray.from_host(x)
+        alg = IF.filter_algorithm(d, (kern,))
+        assert alg == (IF.Algorithm.FFT() if n == 0 else IF.Algorithm.FIR())
+        for k in (kern, off):
+            for b in ("reflect", "circular", IF.Fill(0.5), IF.Fill(np.inf)):
+                got = IF.imfilter(d, k, b)
+                want = IF.imfilter(d, k, b, alg)
+                assert got.eltype is want.eltype
+                np.testing.assert_array_equal(got.to_host(), want.to_host())
+        # the same kernel again on a finite image, its cache entry now in use
+        np.testing.assert_array_equal(IF.imfilter(IF.DeviceArray.from_host(img), kern, "reflect").to_host(),
+                                      IF.imfilter(IF.DeviceArray.from_host(img), kern, "reflect",
+                                                  IF.Algorithm.FFT()).to_host())
