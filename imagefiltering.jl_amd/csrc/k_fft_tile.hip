@@ -27,7 +27,9 @@
 // scalar loads.
 #include <math.h>
 
-#include "ifm_internal.h"
+#include <type_traits>
+
+#include "k_tiles.h"
 
 namespace ifm {
 
@@ -175,20 +177,54 @@ __global__ void __launch_bounds__(TileCfg<F>::NT) k_fft_tile(FftTileArgs a) {
   }
 
   // ---- load both blocks (coalesced along axis 0) into LDS as (A, B) pairs ----
-  bool bad = false;
-  for (int idx = t; idx < F * F; idx += NT) {
-    const int u0 = idx % F, u1 = idx / F;
-    float val[2];
+  // A thread has one column of each block and every RS-th row; its rows are
+  // wave-uniform, and lane l keeps the mapped image row of block rows l, l + 64.
+  // All loads are issued before the first LDS write.  (A border map and an
+  // eltype choice per element took a quarter of the kernel's instructions.)
+  constexpr int RS = NT / F, NI = V;
+  const int u0 = t % F, ub = __builtin_amdgcn_readfirstlane(t / F), lane = t & 63;
+  int col[2], rowm[2][F / 64];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int c = bmap(a.style, a.of0 + x0[s] + a.kf0 + u0, a.n0);
-      const int r = bmap(a.style, a.of1 + y0[s] + a.kf1 + u1, a.n1);
-      val[s] = (c | r) < 0 ? a.fill : load_f(a.in, ioff[s] + c + (int64_t)a.n0 * r, a.dt_in);
-      bad |= !(val[s] - val[s] == 0.f);
-    }
-    lds[u1 * P + u0] = make_float2(val[0], hasB ? val[1] : 0.f);
+  for (int s = 0; s < 2; ++s) {
+    col[s] = bmap(a.style, a.of0 + x0[s] + a.kf0 + u0, a.n0);
+#pragma unroll
+    for (int h = 0; h < F / 64; ++h) rowm[s][h] = bmap(a.style, a.of1 + y0[s] + a.kf1 + lane + 64 * h, a.n1);
   }
-  if (bad) atomicExch(a.nanflag, a.gen);
+  float val[2][NI];
+  const auto load = [&](auto type) {
+    constexpr int DT = decltype(type)::value;
+    uint32_t raw[2][NI];
+    bool in[2][NI];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int u1 = ub + RS * i;
+        const int r = __builtin_amdgcn_readlane(rowm[s][F == 128 && RS * i >= 64 ? F / 64 - 1 : 0], u1 & 63);
+        in[s][i] = (r | col[s]) >= 0;
+        raw[s][i] = raw_ld<DT>(a.in, ioff[s] + (int64_t)a.n0 * max(r, 0) + max(col[s], 0));
+      }
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < NI; ++i) val[s][i] = in[s][i] ? raw_val<DT>(raw[s][i]) : a.fill;
+  };
+  switch (a.dt_in) {
+  case IFM_F32: load(std::integral_constant<int, IFM_F32>()); break;
+  case IFM_F64: load(std::integral_constant<int, IFM_F64>()); break;
+  case IFM_BF16: load(std::integral_constant<int, IFM_BF16>()); break;
+  case IFM_F16: load(std::integral_constant<int, IFM_F16>()); break;
+  case IFM_N0F8: load(std::integral_constant<int, IFM_N0F8>()); break;
+  default: load(std::integral_constant<int, IFM_U8>()); break;
+  }
+  if (!a.skip) {  // otherwise a scan has found every pixel finite
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) bad |= !(val[0][i] - val[0][i] == 0.f) | !(val[1][i] - val[1][i] == 0.f);
+    if (bad) atomicExch(a.nanflag, a.gen);
+  }
+#pragma unroll
+  for (int i = 0; i < NI; ++i) lds[(ub + RS * i) * P + u0] = make_float2(val[0][i], hasB ? val[1][i] : 0.f);
   __syncthreads();
 
   // Task coordinates: tau = t + j NT, line = tau % F, digit = tau / F (wave-uniform).
@@ -318,16 +354,26 @@ __global__ void __launch_bounds__(TileCfg<F>::NT) k_fft_tile(FftTileArgs a) {
   }
   __syncthreads();
   // ---- store the valid outputs of both tiles (coalesced along axis 0) ----
-  for (int idx = t; idx < F * F; idx += NT) {
-    const int u0 = idx % F, u1 = idx / F;
-    if (u0 >= a.T0 || u1 >= a.T1) continue;
-    const float2 r = lds[u1 * P + u0];
+  const auto store = [&](auto *out, auto convert) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       if (s == 1 && !hasB) break;
-      const int c0 = x0[s] + u0, c1 = y0[s] + u1;
-      if (c0 < a.o0 && c1 < a.o1) store_f(a.out, ooff[s] + c0 + (int64_t)a.o0 * c1, a.dt_out, s == 0 ? r.x : r.y);
+      const bool ok = u0 < a.T0 && x0[s] + u0 < a.o0;
+      const int rows = min(a.T1, a.o1 - y0[s]);  // valid rows of the tile
+      auto *p = out + ooff[s] + x0[s] + u0 + (int64_t)a.o0 * (y0[s] + ub);
+#pragma unroll
+      for (int i = 0; i < NI; ++i, p += (int64_t)a.o0 * RS) {
+        if (ub + RS * i >= rows || !ok) continue;
+        const float2 r = lds[(ub + RS * i) * P + u0];
+        *p = convert(s == 0 ? r.x : r.y);
+      }
     }
+  };
+  switch (a.dt_out) {
+  case IFM_F32: store((float *)a.out, [](float v) { return v; }); break;
+  case IFM_F64: store((double *)a.out, [](float v) { return (double)v; }); break;
+  case IFM_BF16: store((uint16_t *)a.out, [](float v) { return f32_to_bf16(v); }); break;
+  default: store((__half *)a.out, [](float v) { return __float2half_rn(v); }); break;
   }
 }
 
