@@ -231,3 +231,26 @@ def test_explicit_padding_too_small_is_dimension_mismatch():
         IF.imfilter(A, kern, IF.Fill(0, (1, 0)))
     with pytest.raises(IF.DimensionMismatch):
         IF.imfilter(A, kern, IF.Fill(0, (0, 0)))
+
+
+def test_factorkernel_rank_pretest_agrees_with_svd():
+    """factorkernel's quick test only ever rejects kernels the SVD rank test
+    rejects: rank one plus perturbations around the tolerance, over scales and
+    shapes."""
+    import sys
+    m = sys.modules["imagefiltering.imfilter"]
+    rng = np.random.default_rng(3)
+    eps = np.sqrt(np.finfo(np.float64).eps)
+    seen = set()
+    for shape in ((2, 2), (3, 5), (7, 7), (21, 15)):
+        for scale in (1e-7, 1e-3, 1.0, 1e6):
+            for level in (0.0, 0.1, 0.9, 1.1, 10.0, 1e3, 1e8):
+                a = scale * np.outer(rng.standard_normal(shape[0]), rng.standard_normal(shape[1]))
+                e = rng.standard_normal(shape)
+                a = a + level * eps * e / np.linalg.norm(e, 2)
+                S = np.linalg.svd(a)[1]
+                separable = all(s < eps for s in S[1:])
+                if m._far_from_rank_one(a):
+                    assert not separable
+                seen.add((m._far_from_rank_one(a), separable))
+    assert (True, False) in seen and (False, True) in seen
