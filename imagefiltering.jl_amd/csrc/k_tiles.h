@@ -155,8 +155,10 @@ __device__ __forceinline__ void sep2d_store(const Sep2dTile &a, const float (&ac
 
 // Axis-0 factor over every staged row of a staged tile (after the staging
 // barrier) into the mid tile; ends with the barrier that publishes it.
+template <int K0 = 0>  // tap count, 0: a.k0
 __device__ __forceinline__ void sep2d_rowpass(const Sep2dTile &a, const float *taps0, float *smem) {
-  const int in_w = S2_TX + a.k0 - 1;
+  const int k0 = K0 ? K0 : a.k0;
+  const int in_w = S2_TX + k0 - 1;
   const int in_h = a.ty + a.k1 - 1;
   const int in_wp = in_w | 1;
   const float *s_in = smem;
@@ -169,8 +171,8 @@ __device__ __forceinline__ void sep2d_rowpass(const Sep2dTile &a, const float *t
     float q[4] = {0.f, 0.f, 0.f, 0.f};
     float w[4] = {src[0], src[1], src[2], 0.f};
     // unrolled so that several LDS reads are in flight
-#pragma unroll 8
-    for (int t = 0; t < a.k0; ++t) {
+#pragma unroll (K0 ? K0 : 8)
+    for (int t = 0; t < k0; ++t) {
       w[3] = src[t + 3];
       const float k = taps0[t];
 #pragma unroll
@@ -187,6 +189,7 @@ __device__ __forceinline__ void sep2d_rowpass(const Sep2dTile &a, const float *t
 // Axis-1 factor over the mid tile for the 32-row band starting at tile row h:
 // each thread owns 8 consecutive rows (h + 8 (t / 64) ..) of column t % 64
 // and slides an 8-value window down the column, one LDS read per tap.
+template <int K1 = 0>  // tap count, 0: a.k1
 __device__ __forceinline__ void sep2d_colpass(const Sep2dTile &a, const float *taps1, const float *smem, int h,
                                               float (&acc)[8]) {
   const float *s_mid = smem + sep2d_mid_offset(a.k0, a.k1, a.ty);
@@ -198,8 +201,9 @@ __device__ __forceinline__ void sep2d_colpass(const Sep2dTile &a, const float *t
   float w[8];
 #pragma unroll
   for (int o = 0; o < 7; ++o) w[o] = src[o * S2_TX];
-#pragma unroll 8
-  for (int t = 0; t < a.k1; ++t) {
+  const int k1 = K1 ? K1 : a.k1;
+#pragma unroll (K1 ? K1 : 8)
+  for (int t = 0; t < k1; ++t) {
     w[7] = src[(t + 7) * S2_TX];
     const float k = taps1[t];
 #pragma unroll
@@ -211,10 +215,11 @@ __device__ __forceinline__ void sep2d_colpass(const Sep2dTile &a, const float *t
 
 // Both factor passes over a staged tile of height S2_TY; on return thread t
 // holds column t % 64, rows 8 (t / 64) .. +7 of the tile.
+template <int K = 0>  // both tap counts, 0: a.k0 and a.k1
 __device__ __forceinline__ void sep2d_filter(const Sep2dTile &a, const float *taps0, const float *taps1,
                                              float *smem, float (&acc)[8]) {
-  sep2d_rowpass(a, taps0, smem);
-  sep2d_colpass(a, taps1, smem, 0, acc);
+  sep2d_rowpass<K>(a, taps0, smem);
+  sep2d_colpass<K>(a, taps1, smem, 0, acc);
 }
 
 // Stages, filters and stores one tile (the caller owns the barrier before
