@@ -1002,7 +1002,9 @@ int ifm_imfilter_default(ifm_ctx *ctx, const ifm_array *in, ifm_array *out, cons
   DenseKernel dk;
   if ((rc = dense_kernel_canon(ctx, kernel, g, in->ndim, dk))) return rc;
   const int F = fft_tile_size(dk);
-  bool ok = in->device && out->device && is_float_out(in->dtype) && F > 0 && dk.n[0] <= 64 && dk.n[1] <= 64 &&
+  // Float64 pixels beyond Float32's range are finite to the scan and not to the
+  // transform: their images are left to the host's choice
+  bool ok = in->device && out->device && is_float_out(in->dtype) && in->dtype != IFM_F64 && F > 0 && dk.n[0] <= 64 && dk.n[1] <= 64 &&
             (b->style != IFM_FILL || isfinite((float)b->fill));
   for (int d = 0; d < in->ndim; ++d) ok = ok && in->size[d] == out->size[d];
   // every pixel lies in its own output's window, so the scan and the

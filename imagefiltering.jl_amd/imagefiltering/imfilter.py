@@ -102,7 +102,7 @@ def factorkernel(kernel):
     m, n = data.shape
     if data.dtype.kind in "iub":
         data = data.astype(np.float64)
-    if data.dtype == np.float64 and _far_from_rank_one(data):
+    if data.dtype == np.float64 and data.size and _far_from_rank_one(data):
         return (k,)
     U, S, Vt = np.linalg.svd(data.astype(np.float64) if data.dtype != np.float32 else data)
     eps = np.sqrt(np.finfo(S.dtype).eps)

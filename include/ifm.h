@@ -184,8 +184,8 @@ int ifm_imfilter_fft(ifm_ctx *ctx, const ifm_array *in, ifm_array *out, const in
  * (src/imfilter.jl:1200-1209) for one dense kernel of more than 30 taps:
  * ifm_imfilter_fft if every pixel is finite, ifm_imfilter_dense (library
  * choice of precision) otherwise, decided on the device, so that the call
- * returns without waiting for the scan of the image.  Device arrays of a
- * floating-point eltype, out of in's size, kernels on axes 0 and 1 of at most
+ * returns without waiting for the scan of the image.  Device arrays of
+ * Float32, BFloat16 or Float16 pixels, out of in's size, kernels on axes 0 and 1 of at most
  * 64 taps that contain their origin, a finite Fill value; IFM_E_UNSUPPORTED
  * otherwise. */
 int ifm_imfilter_default(ifm_ctx *ctx, const ifm_array *in, ifm_array *out, const ifm_kernel *kernel,

@@ -1255,10 +1255,13 @@ def test_default_algorithm_on_device(kshape):
         images.append(x)
     images.append(np.asfortranarray(images[1]))
     images.append(images[3].astype(np.float64))
+    big = img.astype(np.float64)
+    big[5, 5] = 1e300  # finite, but beyond Float32
+    images.append(big)
     for n, x in enumerate(images):
         d = IF.DeviceArray.from_host(x)
         alg = IF.filter_algorithm(d, (kern,))
-        assert alg == (IF.Algorithm.FFT() if n == 0 else IF.Algorithm.FIR())
+        assert alg == (IF.Algorithm.FFT() if np.isfinite(x).all() else IF.Algorithm.FIR())
         for k in (kern, off):
             for b in ("reflect", "circular", IF.Fill(0.5), IF.Fill(np.inf)):
                 got = IF.imfilter(d, k, b)
