@@ -1125,6 +1125,41 @@ def test_iir_line_lengths(n, axis):
                 assert np.max(np.abs(got - want)) <= (tol + extra) * scale, (n, axis, border, T)
 
 
+@pytest.mark.parametrize("sigma", [5.0, 10.0, 20.0])
+@pytest.mark.parametrize("n", [200, 513, 1000, 4097])
+@pytest.mark.parametrize("axis", [0, 1])
+def test_iir_segments_keep_precision(sigma, n, axis):
+    """Lines cut into segments are no less precise than the recursion run
+    element by element: both against the recursion in extended precision.
+
+    Tolerance: the two forms round at the same number of places per value, in a
+    different order; 4 allows for the spread of a norm over 24 random lines."""
+    rng = np.random.default_rng(int(sigma) + n + axis)
+    x = rng.random((n, 24))
+    k = IF.KernelFactors.IIRGaussian(sigma)
+    a, b, M = ([np.longdouble(v) for v in c] for c in (k.a, k.b, np.asarray(k.M).ravel()))
+    y = x.astype(np.longdouble)
+    um, up = y[0] / (1 - sum(a)), y[-1] / (1 - sum(a))
+    h = [um, um, um]
+    for i in range(n):
+        y[i] += a[0] * h[0] + a[1] * h[1] + a[2] * h[2]
+        h = [y[i].copy(), h[0], h[1]]
+    d = [h[i] - up for i in range(3)]
+    vp = up / (1 - sum(b))
+    h = [M[3 * i] * d[0] + M[3 * i + 1] * d[1] + M[3 * i + 2] * d[2] + vp for i in range(3)]
+    y[-1] = h[0]
+    for i in range(n - 2, -1, -1):
+        y[i] += b[0] * h[0] + b[1] * h[1] + b[2] * h[2]
+        h = [y[i].copy(), h[0], h[1]]
+    exact = y * np.longdouble(k.scale)
+    img = np.asfortranarray(x if axis == 0 else x.T)
+    fac = (IF.KernelFactors.ReshapedOneD(2, axis, k),)
+    got = np.asarray(IF.imfilter(IF.Float64, img, fac, "replicate", IF.Algorithm.IIR()))
+    serial = O.imfilter_iir(img, [(axis, k.a, k.b, k.scale, k.M)], "replicate")
+    off = [float(np.linalg.norm((v if axis == 0 else v.T) - exact)) for v in (got, serial)]
+    assert off[0] <= 4 * off[1], off
+
+
 # ---- medians on bit planes -------------------------------------------------------------------
 @pytest.mark.parametrize("k", [3, 5, 7, 9])
 @pytest.mark.parametrize("shape", [(9, 9), (31, 64), (127, 63), (128, 65), (129, 64), (163, 130), (288, 33)])
