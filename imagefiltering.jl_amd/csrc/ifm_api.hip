@@ -1205,12 +1205,17 @@ int ifm_imfilter_iir(ifm_ctx *ctx, const ifm_array *in, ifm_array *out, const if
     } else {
       // Every stage but the first runs in place on one FP64 buffer: the output
       // itself if it is F64.  The last stage writes the output's eltype where
-      // its lines are held in registers.
+      // its lines are held in registers.  in and out may share memory: the
+      // first stage reads in, and writes out only where out is in element for
+      // element (each line's loads precede its stores) or lies elsewhere.
       const auto axis_n = [&](size_t s) { return vi.d.n[g.inv[factors[live[s]].axis]]; };
-      const bool direct = iir_in_registers(axis_n(live.size() - 1));
+      const char *ib = (const char *)vi.d.data, *ob = (const char *)vo.d.data;
+      const bool overlaps = ib < ob + vo.bytes && ob < ib + vi.bytes && !(ib == ob && vi.d.dtype == vo.d.dtype);
+      const bool f64 = vo.d.dtype == IFM_F64;
+      const bool direct = (f64 || iir_in_registers(axis_n(live.size() - 1))) && !(overlaps && live.size() == 1);
       Dense4 buf = vi.d;
       buf.dtype = IFM_F64;
-      if (vo.d.dtype == IFM_F64) {
+      if (f64 && !overlaps) {
         buf.data = vo.d.data;
       } else if (live.size() > 1 || !direct) {
         buf.data = slot_buffer(ctx, S_TMP1, (size_t)cnt * sizeof(double));
@@ -1228,7 +1233,9 @@ int ifm_imfilter_iir(ifm_ctx *ctx, const ifm_array *in, ifm_array *out, const if
         for (int i = 0; i < 9; ++i) c.M[i] = k.M[i];
         HIPCHK(launch_iir(src, dst, g.inv[k.axis], c, isfill, b->fill, st));
       }
-      if (!direct && buf.data != vo.d.data) {
+      if (!direct && f64) {
+        HIPCHK(hipMemcpyAsync(vo.d.data, buf.data, vo.bytes, hipMemcpyDeviceToDevice, st));
+      } else if (!direct) {
         FirPass p;
         p.axis = 0;
         p.len = 1;

@@ -1160,6 +1160,42 @@ def test_iir_segments_keep_precision(sigma, n, axis):
     assert off[0] <= 4 * off[1], off
 
 
+@pytest.mark.parametrize("n", [300, 8200])
+@pytest.mark.parametrize("ein,eout,shift", [("Float64", "Float32", 0), ("Float32", "Float64", 0), ("Float32", "Float32", 0),
+                                            ("Float64", "Float64", 0), ("Float32", "Float32", 24), ("Float64", "Float64", 40),
+                                            ("Float32", "BFloat16", 0), ("BFloat16", "Float64", 16)])
+def test_iir_in_and_out_share_memory(n, ein, eout, shift):
+    """in and out of ifm_imfilter_iir may alias: in one block of memory (out
+    `shift` elements after in), of equal and of different eltypes, one to three
+    factors, lines in registers and longer ones: the bits of the call on
+    separate arrays."""
+    from imagefiltering import _lib
+    from imagefiltering.device import ifm_array
+    from imagefiltering.imfilter import _border_struct
+    L, ctx = _lib.load(), _lib.ctx()
+    ein, eout = getattr(IF, ein), getattr(IF, eout)
+    k = IF.KernelFactors.IIRGaussian(3.0)
+    for shape, axes in (((n, 23), (0,)), ((23, n), (1,)), ((n, 23), (0, 1)), ((23, n), (0, 1)), ((23, n), (0, 1, 0))):
+        fa = (_lib.IfmIir * len(axes))()
+        for f, axis in zip(fa, axes):
+            f.axis, f.scale = axis, k.scale
+            f.a[:], f.b[:], f.M[:] = list(k.a), list(k.b), [float(m) for m in np.asarray(k.M).ravel()]
+        b = _border_struct(IF.borderinstance("replicate"), ein)
+        cnt = shape[0] * shape[1]
+        src, want = IF.DeviceArray(shape, ein), IF.DeviceArray(shape, eout)
+        _lib.check(L.ifm_fill_uniform(ctx, ifm_array(src), 5))
+        host = np.asfortranarray(np.asarray(src.to_host()))
+        _lib.check(L.ifm_imfilter_iir(ctx, ifm_array(src), ifm_array(want), fa, len(axes), b))
+        block = IF.DeviceArray((8 * cnt + 8 * shift,), IF.UInt8)
+        _lib.check(L.ifm_memcpy_h2d(ctx, block.ptr, host.ctypes.data, host.nbytes))
+        a, o = ifm_array(src), ifm_array(want)
+        a.data, o.data = block.ptr, block.ptr + shift * eout.itemsize
+        _lib.check(L.ifm_imfilter_iir(ctx, a, o, fa, len(axes), b))
+        got = np.empty(shape, dtype=eout.storage, order="F")
+        _lib.check(L.ifm_memcpy_d2h(ctx, got.ctypes.data, o.data, got.nbytes))
+        np.testing.assert_array_equal(got, np.asarray(want.to_host()), err_msg="%r %r" % (shape, axes))
+
+
 # ---- medians on bit planes -------------------------------------------------------------------
 @pytest.mark.parametrize("k", [3, 5, 7, 9])
 @pytest.mark.parametrize("shape", [(9, 9), (31, 64), (127, 63), (128, 65), (129, 64), (163, 130), (288, 33)])
