@@ -1011,6 +1011,13 @@ int ifm_imfilter_default(ifm_ctx *ctx, const ifm_array *in, ifm_array *out, cons
   // transform see the same pixels
   for (int m = 0; m < 2; ++m) ok = ok && dk.first[m] <= 0 && dk.first[m] + dk.n[m] > 0;
   if (!ok) return fail(ctx, IFM_E_UNSUPPORTED, "ifm_imfilter_default: not a tiled 2-D transform of a device array");
+  // A graph would replay this call's flag generation (one replay that met a NaN
+  // would decide all later ones) and keep the cache entry's address.
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return fail(ctx, IFM_E_UNSUPPORTED, "ifm_imfilter_default: the stream is being captured");
+  }
   View vi, vo;
   if ((rc = make_view(ctx, in, g, S_IN, true, vi))) return rc;
   if ((rc = make_view(ctx, out, g, S_OUT, false, vo))) return rc;

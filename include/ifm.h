@@ -185,9 +185,9 @@ int ifm_imfilter_fft(ifm_ctx *ctx, const ifm_array *in, ifm_array *out, const in
  * ifm_imfilter_fft if every pixel is finite, ifm_imfilter_dense (library
  * choice of precision) otherwise, decided on the device, so that the call
  * returns without waiting for the scan of the image.  Device arrays of
- * Float32, BFloat16 or Float16 pixels, out of in's size, kernels on axes 0 and 1 of at most
- * 64 taps that contain their origin, a finite Fill value; IFM_E_UNSUPPORTED
- * otherwise. */
+ * Float32, BFloat16 or Float16 pixels, out of in's size, kernels on axes 0 and
+ * 1 of at most 64 taps that contain their origin, a finite Fill value, a
+ * stream that is not being captured into a graph; IFM_E_UNSUPPORTED otherwise. */
 int ifm_imfilter_default(ifm_ctx *ctx, const ifm_array *in, ifm_array *out, const ifm_kernel *kernel,
                          const ifm_border *border);
 

@@ -1343,3 +1343,40 @@ def test_default_algorithm_on_device(kshape):
         np.testing.assert_array_equal(IF.imfilter(IF.DeviceArray.from_host(img), kern, "reflect").to_host(),
                                       IF.imfilter(IF.DeviceArray.from_host(img), kern, "reflect",
                                                   IF.Algorithm.FFT()).to_host())
+
+
+def test_default_algorithm_is_not_captured():
+    """The device's choice is refused on a stream under graph capture: a replay
+    would decide by the flag of an earlier one.  The capture itself stays valid,
+    and the same call runs before and after it."""
+    import ctypes as C
+    from imagefiltering import _lib
+    from imagefiltering.device import ifm_array
+    from imagefiltering.imfilter import _border_struct, _kernel_struct
+    L = _lib.load()
+    _lib.ctx()
+    rng = np.random.default_rng(1)
+    d = IF.DeviceArray.from_host(rng.random((150, 133)).astype(np.float32))
+    kern = IF.centered(rng.standard_normal((9, 9)))
+    want = IF.imfilter(d, kern, "reflect").to_host()
+    out = IF.DeviceArray(d.shape, IF.Float64, d.order)
+    st, ctx, graph = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert L.hipStreamCreate(C.byref(st)) == 0
+    assert L.ifm_ctx_create(0, st, C.byref(ctx)) == 0
+    args = (ctx, ifm_array(d), ifm_array(out), _kernel_struct(kern), _border_struct(IF.borderinstance("reflect"), IF.Float32))
+    try:
+        assert L.ifm_imfilter_default(*args) == 0
+        assert L.ifm_ctx_synchronize(ctx) == 0
+        assert L.hipStreamBeginCapture(st, 1) == 0  # thread-local capture mode
+        rc = L.ifm_imfilter_default(*args)
+        assert L.hipStreamEndCapture(st, C.byref(graph)) == 0
+        assert rc == _lib.E_UNSUPPORTED
+        assert L.ifm_memset_d(ctx, out.ptr, 255, out.nbytes) == 0
+        assert L.ifm_imfilter_default(*args) == 0
+        assert L.ifm_ctx_synchronize(ctx) == 0
+        np.testing.assert_array_equal(out.to_host(), want)
+    finally:
+        if graph:
+            L.hipGraphDestroy(graph)
+        L.ifm_ctx_destroy(ctx)
+        L.hipStreamDestroy(st)
