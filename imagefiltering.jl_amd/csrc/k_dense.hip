@@ -86,9 +86,11 @@ struct Dense2dArgs {
   Gate gate;
 };
 
+template <bool GATED>
 __global__ void __launch_bounds__(256) k_dense2d_valu(Dense2dArgs a) {
   extern __shared__ float smem[];
-  if (gate_closed(a.gate)) return;
+  if constexpr (GATED)
+    if (gate_closed(a.gate)) return;
   const int IN_W = DV_TX + a.k0 - 1;
   const int IN_H = DV_TY + a.k1 - 1;
   const int IN_WP = IN_W | 1;
@@ -157,13 +159,14 @@ struct SmallTaps {
   float k[KX * KY];  // column-major (axis 0 fastest)
 };
 
-template <int KX, int KY>
+template <int KX, int KY, bool GATED>
 __global__ void __launch_bounds__(256) k_dense2d_small(Dense2dArgs a, SmallTaps<KX, KY> kt) {
   constexpr int IN_W = DV_TX + KX - 1, IN_H = DV_TY + KY - 1, IN_WP = IN_W | 1;
   constexpr int NE = IN_H * IN_W, NI = (NE + 255) / 256;
   __shared__ float smem[IN_H * IN_WP];
   __shared__ int smap[IN_H + IN_W];  // border tiles: source row of tile row r, then source column of tile column c
-  if (gate_closed(a.gate)) return;
+  if constexpr (GATED)
+    if (gate_closed(a.gate)) return;
   const int tid = threadIdx.x;
   const int tx = tid & 63, ty = tid >> 6;
   const int tile = xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
@@ -255,11 +258,19 @@ __global__ void __launch_bounds__(256) k_dense2d_small(Dense2dArgs a, SmallTaps<
   }
 }
 
+// The test of the gate is left out of plain launches where it costs: it waits for
+// the arguments and branches before the staging loads go out.  3 x 3 / 5 x 5 /
+// 7 x 7 F32: 4.75 / 5.10 / 6.05 us with it, 4.44 / 4.81 / 5.80 without
+// (1000 x 800), 19.1 / 23.1 / 35.8 and 18.6 / 22.7 / 35.1 (4001 x 3001); 4 x 4
+// in k_dense2d_valu 22.3 and 22.0.  From 9 x 9 on it costs nothing: 50.0 with,
+// 50.5 without (9 x 9), 115.2 and 115.7 (13 x 13).
 template <int KX, int KY>
 static hipError_t launch_small(const Dense2dArgs &a, const float *taps, dim3 grid, hipStream_t st) {
   SmallTaps<KX, KY> kt;
   for (int i = 0; i < KX * KY; ++i) kt.k[i] = taps[i];
-  hipLaunchKernelGGL((k_dense2d_small<KX, KY>), grid, dim3(256), 0, st, a, kt);
+  constexpr bool PLAIN = KX * KY <= 49;
+  if (PLAIN && !a.gate.flag) hipLaunchKernelGGL((k_dense2d_small<KX, KY, !PLAIN>), grid, dim3(256), 0, st, a, kt);
+  else hipLaunchKernelGGL((k_dense2d_small<KX, KY, true>), grid, dim3(256), 0, st, a, kt);
   return hipGetLastError();
 }
 
@@ -522,7 +533,8 @@ hipError_t launch_dense_valu(const Dense4 &in, Dense4 &out, const int64_t *out_f
       default: return launch_small_ky<15>(a.k1, a, taps, grid, st);
       }
     }
-    hipLaunchKernelGGL(k_dense2d_valu, grid, dim3(256), lds, st, a);
+    if (a.gate.flag) hipLaunchKernelGGL(k_dense2d_valu<true>, grid, dim3(256), lds, st, a);
+    else hipLaunchKernelGGL(k_dense2d_valu<false>, grid, dim3(256), lds, st, a);
     return hipGetLastError();
   }
   if (gate.flag) return hipErrorInvalidValue;  // 2-D kernels of up to 64 taps per axis only

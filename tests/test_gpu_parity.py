@@ -1380,3 +1380,21 @@ def test_default_algorithm_is_not_captured():
             L.hipGraphDestroy(graph)
         L.ifm_ctx_destroy(ctx)
         L.hipStreamDestroy(st)
+
+
+@pytest.mark.parametrize("kshape", [(3, 11), (11, 3), (7, 7), (3, 15), (9, 7), (9, 9), (13, 5), (15, 13), (4, 9), (64, 3)])
+def test_default_algorithm_direct_sums(kshape):
+    """The direct sums behind the default algorithm's gate, at the kernel sizes
+    where their plain launches leave the gate's test out or keep it: run where a
+    pixel is not finite, leaving the transform's output alone where all are."""
+    rng = np.random.default_rng(kshape[0] * 100 + kshape[1])
+    kern = IF.centered(rng.standard_normal(kshape))
+    img = rng.random((150, 133)).astype(np.float32)
+    for at in (None, (149, 132), None, (0, 0)):
+        x = img.copy()
+        if at is not None:
+            x[at] = np.nan
+        d = IF.DeviceArray.from_host(x)
+        alg = IF.Algorithm.FFT() if at is None else IF.Algorithm.FIR()
+        np.testing.assert_array_equal(IF.imfilter(d, kern, "reflect").to_host(),
+                                      IF.imfilter(d, kern, "reflect", alg).to_host())
