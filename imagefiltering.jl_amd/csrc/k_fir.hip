@@ -348,6 +348,43 @@ static int march_rows(int64_t o1, int64_t strips, int k) {
 // taps beyond 13.
 constexpr int64_t SM_PIXELS = 4000000, SM_BATCH_PIXELS = 16000000;
 
+// Above that line the speed over tiles is estimated from what it was measured
+// to depend on (816 shapes: 20 to 4096 columns in one plane and in stacks, 3 to
+// 33 taps, F32, bf16 and N0f8, 1 to 3 times the line; what marches by this rule
+// was at worst 0.93 of the tiles' speed, and 0.53 before there was one):
+//  * columns: the filled part of 128-column strips against that of 64-column
+//    tiles.  13 taps, N0f8: 60 x 90000 24.7 us in tiles, 33.2 marched; 4096 wide
+//    and as large 26.3 and 26.6.
+//  * rows: planes that do not fill 32-row tiles, against the K - 1 rows before
+//    each chunk.  33 taps F32: planes of 64 x 30 87 and 136, of 500 x 33 153 and
+//    78.
+//  * size, by the strips' pixels: 33 taps F32 1.09 times as fast at the line, 1.5
+//    at three times that.
+//  * eltype: single elements of 1 and 2 bytes are loaded where F32 comes in
+//    pairs.  21 taps bf16: 0.85 at the line, 1.10 at three times that.
+struct MarchFill {
+  double columns, cover;  // 64-column tiles and the half strips over them
+  double tiled, marched;  // rows of the tiles, and of chunks with what precedes them over that of a full chunk
+  MarchFill(int k, int64_t o0, int64_t o1, int rows) {
+    columns = (double)((o0 + S2_TX - 1) / S2_TX);
+    cover = (double)((o0 + SM_W - 1) / SM_W * 2);
+    tiled = (double)((o1 + S2_TY - 1) / S2_TY * S2_TY * (rows + k - 1));
+    marched = (double)((o1 + (o1 + rows - 1) / rows * (k - 1)) * rows);
+  }
+};
+static double march_eltype(int dt, double one_byte, double two_bytes) {
+  return dt == IFM_F32 ? 1.0 : dt == IFM_BF16 || dt == IFM_F16 ? two_bytes : one_byte;
+}
+
+bool sep_march_pays(int k, int dt_in, int64_t o0, int64_t o1, int64_t nplanes) {
+  const double line = (double)SM_PIXELS * std::max(k, 13) / 13;
+  if ((double)o0 * o1 * nplanes < line) return false;
+  const double size = (double)SM_W * ((o0 + SM_W - 1) / SM_W) * o1 * nplanes / line;
+  const double speed = (k <= 5 ? 1.5 : k <= 9 ? 1.2 : 1.05) + std::min(0.35, 0.18 * (size - 1));
+  const MarchFill f(k, o0, o1, SM_MAXROWS);
+  return speed * march_eltype(dt_in, 0.92, 0.82) * (0.25 * f.cover + 0.75 * f.columns) * f.tiled >= f.cover * f.marched;
+}
+
 static bool sep_march_takes(int k0, int k1, int dt_in) {
   const bool k = k0 == 3 || k0 == 5 || k0 == 7 || k0 == 9 || k0 == 13 || k0 == 17 || k0 == 21 || k0 == 25 || k0 == 29 ||
                  k0 == 33;
@@ -362,8 +399,7 @@ static bool march_launch(const Sep2dArgs &s, hipStream_t st) {
   m.rows = march_rows(s.o1, (int64_t)m.strips * s.nplanes, s.k0);
   m.chunks = (s.o1 + m.rows - 1) / m.rows;
   m.waves = (int64_t)m.strips * m.chunks * s.nplanes;
-  if ((int64_t)s.o0 * s.o1 * s.nplanes * 13 < SM_PIXELS * std::max(s.k0, 13) || m.waves > (int64_t(1) << 31))
-    return false;
+  if (!sep_march_pays(s.k0, s.dt_in, s.o0, s.o1, s.nplanes) || m.waves > (int64_t(1) << 31)) return false;
   const dim3 grid((unsigned)((m.waves + 3) / 4));
   switch (s.k0) {
 #define MARCH(K) \
@@ -702,14 +738,20 @@ __global__ void __launch_bounds__(256) k_sep_march_batch(const SepReq *__restric
 // longest factors) and end with its longest waves, so the line is drawn higher
 // than for one image.  Batches of the serving mix (sides up to 2048), in tiles
 // and marched: 24 requests 143 / 172 us, 48: 231 / 246, 96: 441 / 393, 256: 830
-// / 715.
-bool sep_march_batched(int k0, int k1, int dt_in, int64_t batch_pixels) {
-  return sep_march_takes(k0, k1, dt_in) && batch_pixels * 13 >= SM_BATCH_PIXELS * std::max(k0, 13);
+// / 715.  Above it the request's own shape and eltype decide, as for one image:
+// 1000 of 60 x 300, 9 taps: F32 95 / 135, bf16 81 / 171; 300 of 300 x 200: 101 /
+// 102 and 81 / 121; 200 of 512 x 200: 100 / 88 and 83 / 95.
+constexpr int SM_BATCH_ROWS = 32;  // rows per chunk
+bool sep_march_batched(int k0, int k1, int dt_in, int64_t n0, int64_t n1, int64_t batch_pixels) {
+  if (!sep_march_takes(k0, k1, dt_in) || batch_pixels * 13 < SM_BATCH_PIXELS * std::max(k0, 13)) return false;
+  const double speed = k0 <= 9 ? 1.27 : k0 < 21 ? 1.3 : 1.5;
+  const MarchFill f(k0, n0, n1, SM_BATCH_ROWS);
+  return speed * march_eltype(dt_in, 0.8, 0.7) * f.columns * f.tiled >= f.cover * f.marched;
 }
 
 // Workgroups of a marched request, and its rows per chunk.
 int sep_march_groups(int n0, int n1, int *rows) {
-  *rows = 32;
+  *rows = SM_BATCH_ROWS;
   const int64_t waves = (int64_t)((n0 + SM_W - 1) / SM_W) * ((n1 + *rows - 1) / *rows);
   return (int)((waves + 3) / 4);
 }

@@ -1307,6 +1307,107 @@ def test_fir_march_equals_tiles(k, shape):
             np.testing.assert_array_equal(np.asarray(got.data)[:, :, z], np.asarray(one.data))
 
 
+@pytest.mark.parametrize("k", [3, 5, 7, 9, 13, 17, 21, 25, 29, 33])
+def test_fir_march_strips(k):
+    """Planes of three whole strips and a ragged one, two chunks and more of
+    rows: border strips, strips loaded in unaligned pairs (interior ones of F32)
+    and Fill rows above and below those.  Bit for bit the planes filtered alone,
+    in tiles."""
+    import ctypes as C
+    from imagefiltering import _lib
+    pays = _lib.load()._ZN3ifm14sep_march_paysEiilll
+    pays.argtypes, pays.restype = [C.c_int, C.c_int] + [C.c_int64] * 3, C.c_bool
+    rng = np.random.default_rng(k)
+    shape = (421, 70)
+    taps = [rng.standard_normal(k), rng.standard_normal(k)]
+    planes = int(2.4 * 4_000_000 * max(k, 13) / 13 / (shape[0] * shape[1]))
+    some = [0, planes // 2, planes - 1]
+
+    def kern(n):
+        return tuple(IF.KernelFactors.ReshapedOneD(n, d, IF.centered(taps[d])) for d in range(2))
+
+    vol = np.asfortranarray(rng.random(shape + (planes,), dtype=np.float32) - 0.5)
+    codes = np.asfortranarray(rng.integers(0, 256, shape + (planes,), dtype=np.uint8))
+    for a, b, T in ((vol, IF.Fill(0.5), IF.Float32), (vol, "reflect", IF.Float64),
+                    (vol.astype(np.float16), "circular", IF.Float32), (codes, "symmetric", IF.Float32)):
+        dt = IF.eltypes.eltype_of(a).code
+        assert pays(k, dt, *shape, planes) and not pays(k, dt, *shape, 1)
+        got = IF.imfilter(T, IF.DeviceArray.from_host(a), kern(3), b, IF.Algorithm.FIRTiled()).to_host()
+        for z in some:
+            one = np.asarray(IF.imfilter(T, np.asfortranarray(a[:, :, z]), kern(2), b, IF.Algorithm.FIRTiled()))
+            np.testing.assert_array_equal(got[:, :, z], one)
+
+
+def _separable_request(shape, et, oet, k, border, seed, k1=None, second=False):
+    """A separable batch request on a filled device image, and its arrays."""
+    import ctypes as C
+    from imagefiltering import _lib
+    from imagefiltering.device import ifm_array
+    from imagefiltering.imfilter import _border_struct
+    rng = np.random.default_rng(seed)
+    src, out = IF.DeviceArray(shape, et), IF.DeviceArray(shape, oet)
+    _lib.check(_lib.load().ifm_fill_uniform(_lib.ctx(), ifm_array(src), seed))
+    q = _lib.IfmRequest()
+    q.op, q.in_, q.out, q.border = _lib.OP_SEPARABLE, ifm_array(src), ifm_array(out), _border_struct(
+        IF.borderinstance(border), et)
+    outs, taps = [out], []
+    for fs, count in ((q.factors, "nfactors"), (q.factors2, "nfactors2"))[: 2 if second else 1]:
+        setattr(q, count, 2)
+        for axis, n in ((0, k), (1, k1 or k)):
+            taps.append(rng.standard_normal(n))
+            fs[axis].axis, fs[axis].len, fs[axis].first = axis, n, -(n // 2)
+            fs[axis].taps = taps[-1].ctypes.data_as(C.POINTER(C.c_double))
+    if second:
+        outs.append(IF.DeviceArray(shape, oet))
+        q.out2 = ifm_array(outs[1])
+    return q, outs, (src, taps)
+
+
+def test_marched_batch_equals_requests_alone():
+    """A batch above the marching line, with every marched length, requests that
+    stay in tiles beside them (other lengths, narrow images, 16-bit pixels),
+    small ones whose strips and chunks are ragged, two outputs, every border: bit
+    for bit the same requests run alone, below the line."""
+    import ctypes as C
+    from imagefiltering import _lib
+    L, ctx = _lib.load(), _lib.ctx()
+    marched = L._ZN3ifm17sep_march_batchedEiiilll
+    marched.argtypes, marched.restype = [C.c_int] * 3 + [C.c_int64] * 3, C.c_bool
+    borders = STYLES + [IF.Fill(0.25)]
+    specs = []  # shape, eltype, output eltype, lengths, two outputs
+    for i, k in enumerate((3, 5, 7, 9, 13, 17, 21, 25, 29, 33)):
+        specs.append(((2100, 2003), IF.BFloat16 if k in (21, 33) else IF.Float32, IF.Float32, k, k, False))
+        specs.append(((421, 70 + k), IF.Float32, IF.Float64, k, k, False))
+        specs.append(((130 - i, 16 + i), IF.Float32, IF.Float64, k, k, k == 3))
+    specs += [((61, 300), IF.Float32, IF.Float32, 9, 9, False), ((255, 97), IF.BFloat16, IF.Float32, 5, 5, False),
+              ((300, 200), IF.Float32, IF.Float32, 11, 11, False), ((300, 200), IF.Float32, IF.Float64, 9, 13, True),
+              ((1, 1), IF.Float32, IF.Float32, 3, 3, False)]
+    px = sum(s[0] * s[1] * (2 if two else 1) for s, *_, two in specs)
+    took = [marched(k0, k1, et.code, *shape, px) for shape, et, _, k0, k1, _ in specs]
+    assert sum(took) >= 20 and not all(took)
+    assert {s[3] for s, m in zip(specs, took) if m and s[1] is IF.Float32 and s[0][0] == 421} >= {3, 5, 7, 9, 13, 17, 21}
+    reqs, outs, keep = [], [], []
+    for i, (shape, et, oet, k0, k1, two) in enumerate(specs):
+        b = borders[i % 5] if min(shape) > 1 else "replicate"
+        q, o, x = _separable_request(shape, et, oet, k0, b, 100 + i, k1, two)
+        reqs.append(q)
+        outs.append(o)
+        keep.append(x)
+        one = (_lib.IfmRequest * 1)(q)
+        assert not marched(k0, k1, et.code, *shape, shape[0] * shape[1] * (2 if two else 1))
+        _lib.check(L.ifm_batch_run(ctx, one, 1))
+    _lib.check(L.ifm_ctx_synchronize(ctx))
+    alone = [[d.to_host() for d in o] for o in outs]
+    for o in outs:
+        for d in o:
+            _lib.check(L.ifm_memset_d(ctx, d.ptr, 255, d.nbytes))
+    _lib.check(L.ifm_batch_run(ctx, (_lib.IfmRequest * len(reqs))(*reqs), len(reqs)))
+    _lib.check(L.ifm_ctx_synchronize(ctx))
+    for i, o in enumerate(outs):
+        for d, want in zip(o, alone[i]):
+            np.testing.assert_array_equal(d.to_host(), want, err_msg="request %d: %r" % (i, specs[i]))
+
+
 # ---- the default algorithm of one long dense kernel, chosen on the device ----------------------
 @pytest.mark.parametrize("kshape", [(7, 7), (8, 6), (15, 15), (21, 17), (31, 31), (33, 20), (45, 45)])
 def test_default_algorithm_on_device(kshape):

@@ -254,3 +254,50 @@ def test_factorkernel_rank_pretest_agrees_with_svd():
                     assert not separable
                 seen.add((m._far_from_rank_one(a), separable))
     assert (True, False) in seen and (False, True) in seen
+
+
+# ---- dispatch rules of the library (host functions, no GPU) --------------------------------------
+U8, N0F8, F32, F64, BF16, F16 = range(6)  # eltype codes
+
+
+def test_separable_march_rule():
+    """Which equal pairs of factors march down 128-column strips: wide images
+    above the size line, by eltype; not narrow ones, whose strips would be half
+    empty, in one plane or in a stack."""
+    import ctypes as C
+    from imagefiltering import _lib
+    pays = _lib.load()._ZN3ifm14sep_march_paysEiilll
+    pays.argtypes, pays.restype = [C.c_int, C.c_int] + [C.c_int64] * 3, C.c_bool
+    for k in (3, 5, 7, 9, 13, 17, 21, 25, 29, 33):
+        line = 4_000_000 * max(k, 13) // 13
+        for dt in (U8, N0F8, F32, BF16, F16):
+            assert not pays(k, dt, 4096, line // 4096 - 1, 1)
+            assert pays(k, dt, 4096, 4 * line // 4096, 1)
+            assert pays(k, dt, 512, 128, 4 * line // (512 * 128))
+            if k > 5 or dt in (BF16, F16):
+                assert not pays(k, dt, 60, 4 * line // 60, 1)
+                assert not pays(k, dt, 64, 64, 4 * line // 4096)
+            # every size above one that marches marches too
+            took = [pays(k, dt, 300, line * f // 1200, 1) for f in range(4, 20)]
+            assert took == sorted(took)
+        assert pays(k, F32, 4096, line // 4096 + 1, 1)
+    assert not pays(21, BF16, 4096, 6_500_000 // 4096 + 1, 1)
+
+
+def test_separable_march_rule_of_batches():
+    import ctypes as C
+    from imagefiltering import _lib
+    marched = _lib.load()._ZN3ifm17sep_march_batchedEiiilll
+    marched.argtypes, marched.restype = [C.c_int] * 3 + [C.c_int64] * 3, C.c_bool
+    big = 1 << 28
+    for k in (3, 5, 7, 9, 13, 17, 21, 25, 29, 33):
+        line = 16_000_000 * max(k, 13) // 13
+        assert not marched(k, k, F32, 1024, 1024, line - 1)
+        assert marched(k, k, F32, 1024, 1024, line + 1)
+        assert not marched(k, k, F64, 1024, 1024, big)
+        assert not marched(k, k + 2, F32, 1024, 1024, big)
+        for dt in (N0F8, F32, BF16):
+            assert not marched(k, k, dt, 60, 300, big)
+            assert not marched(k, k, dt, 64, 64, big)
+        assert marched(k, k, BF16, 1024, 1024, big) == (k >= 21)
+    assert not marched(11, 11, F32, 1024, 1024, big)
