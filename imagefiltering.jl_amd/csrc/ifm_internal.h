@@ -402,6 +402,8 @@ hipError_t launch_sep_march_batch(const SepReq *reqs, const int *tile_req, const
 hipError_t launch_sep_batch(const SepReq *reqs, const int *tile_req, const int *tile_first, int ntiles,
                             size_t lds_bytes, hipStream_t st);
 void median_batch_tile(int k, bool pack, int *bx, int *by);
+// Whether a median of codes is taken on bit planes.
+bool median_on_bits(int k, int64_t o0, int64_t o1, int64_t nplanes);
 uint32_t median_fill_key(int dt, double fill);
 hipError_t launch_median_batch(int k, bool pack, const MedianArgs *reqs, const int *tile_req, const int *tile_first,
                                int ntiles, hipStream_t st);

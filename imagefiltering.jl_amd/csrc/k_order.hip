@@ -1047,12 +1047,20 @@ hipError_t launch_median_band_batch(int k, const BandJob *jobs, const int *tile_
 // than one network tile (its 8 planes are a serial chain), so below about one
 // tile per CU the network is faster for K = 5 and 7: 1024^2 (128 tiles) 6.7 /
 // 9.3 us against 8.5 / 11.3; 1448^2 (276 tiles) 10.9 / 18.0 against 9.8 /
-// 13.2; 8192^2 162 / 326 against 75 / 123.  K = 3: 724^2 8.5 against 6.6,
+// 13.2; 8192^2 162 / 326 against 75 / 123.  Above that, a tile counts whether it
+// is filled or not, so planes that leave the 128 x 64 tiles part empty are
+// weighed by the network tiles they take: 2000 planes of 24 x 24 15.0 / 25.6
+// against 26.5 / 39.9; 300 of 64 x 64 8.1 / 11.7 against 10.1 / 13.8; 200 of 100 x
+// 100 14.0 / 22.9 against 10.4 / 14.7.  (The two lines through the times of 42
+// stacks, 200 to 3000 tiles.)  K = 3: no slower anywhere; 724^2 8.5 against 6.6,
 // 8192^2 109 against 51.
-static bool median_on_bits(const MedianArgs &a, bool codes, int k) {
-  if (!codes || a.fillkey > 0xffu) return false;
-  const int64_t tiles = (int64_t)((a.o0 + MB_BX - 1) / MB_BX) * ((a.o1 + MB_BY - 1) / MB_BY) * a.nplanes;
-  return k == 3 || k == 9 || tiles >= 192;
+bool median_on_bits(int k, int64_t o0, int64_t o1, int64_t nplanes) {
+  if (k == 3 || k == 9) return true;
+  const int64_t tiles = (o0 + MB_BX - 1) / MB_BX * ((o1 + MB_BY - 1) / MB_BY) * nplanes;
+  int bx, by;
+  median_batch_tile(k, true, &bx, &by);
+  const int64_t net = (o0 + bx - 1) / bx * ((o1 + by - 1) / by) * nplanes;
+  return tiles >= 192 && (k == 5 ? net > 280 + 2.1 * tiles : net > 160 + 1.75 * tiles);
 }
 
 hipError_t launch_median(const Dense4 &in, Dense4 &out, const int64_t *out_first, const int *wfirst,
@@ -1095,7 +1103,7 @@ hipError_t launch_median(const Dense4 &in, Dense4 &out, const int64_t *out_first
       else if (k == 5) launch_f64<5, 2, 2>(a, fill, st);
       else if (k == 7) launch_f64<7, 2, 2>(a, fill, st);
       else launch_f64<9, 2, 2>(a, fill, st);
-    } else if (median_on_bits(a, codes, k)) {
+    } else if (codes && a.fillkey <= 0xffu && median_on_bits(k, a.o0, a.o1, a.nplanes)) {
       if (k == 3) launch_bits<3>(a, st);
       else if (k == 5) launch_bits<5>(a, st);
       else if (k == 7) launch_bits<7>(a, st);

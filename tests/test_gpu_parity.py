@@ -1235,6 +1235,29 @@ def test_median_codes_tile_edges(k, shape):
             np.testing.assert_array_equal(np.asarray(inner)[:, :, z], want[h:shape[0] - h, h:shape[1] - h])
 
 
+@pytest.mark.parametrize("k", [5, 7])
+@pytest.mark.parametrize("shape,planes", [((127, 63), 192), ((128, 65), 160), ((129, 64), 160), ((163, 130), 130),
+                                          ((288, 33), 90), ((100, 41), 192), ((64, 64), 700)])
+def test_median_codes_tile_edges_in_stacks(k, shape, planes):
+    """The same edges on stacks that the 5 x 5 and 7 x 7 bit planes are taken for,
+    and a stack of half-empty tiles on either side of the line: bit-exact."""
+    import ctypes as C
+    from imagefiltering import _lib
+    bits = _lib.load()._ZN3ifm14median_on_bitsEilll
+    bits.argtypes, bits.restype = [C.c_int] + [C.c_int64] * 3, C.c_bool
+    assert bits(k, *shape, planes) == (shape != (64, 64) or k == 7)
+    rng = np.random.default_rng(k * 1000 + shape[0])
+    h = k // 2
+    vol = rng.integers(0, 256, shape + (planes,)).astype(np.uint8)
+    vol[:, :, ::2] %= 3                                  # ties
+    vol = np.asfortranarray(vol)
+    for b in STYLES + [IF.Fill(7)]:
+        got = np.asarray(IF.mapwindow(IF.median_, vol, (k, k, 1), border=b))
+        for z in (0, 1, planes - 1):
+            want = O.median(vol[:, :, z].astype(np.float64), [-h, -h], [k, k], obord(b))
+            np.testing.assert_array_equal(got[:, :, z], want)
+
+
 # ---- Float64 medians and 9 x 9 windows ---------------------------------------------------------
 @pytest.mark.parametrize("k", [3, 5, 7, 9])
 @pytest.mark.parametrize("shape", [(9, 9), (63, 17), (65, 16), (129, 33)])

@@ -301,3 +301,22 @@ def test_separable_march_rule_of_batches():
             assert not marched(k, k, dt, 64, 64, big)
         assert marched(k, k, BF16, 1024, 1024, big) == (k >= 21)
     assert not marched(11, 11, F32, 1024, 1024, big)
+
+
+def test_median_bit_plane_rule():
+    """Medians of codes: 5 x 5 and 7 x 7 windows take bit planes where the images
+    fill enough 128 x 64 tiles, in one plane or in a stack; not stacks of planes
+    that leave the tiles mostly empty, however many."""
+    import ctypes as C
+    from imagefiltering import _lib
+    bits = _lib.load()._ZN3ifm14median_on_bitsEilll
+    bits.argtypes, bits.restype = [C.c_int] + [C.c_int64] * 3, C.c_bool
+    for k in (3, 9):
+        assert bits(k, 9, 9, 1) and bits(k, 24, 24, 2000)
+    for k in (5, 7):
+        assert not bits(k, 1024, 1024, 1) and bits(k, 1448, 1448, 1) and bits(k, 8192, 8192, 1)
+        assert bits(k, 100, 100, 200) and bits(k, 300, 300, 60)
+        for planes in (200, 2000, 100000):
+            assert not bits(k, 24, 24, planes) and not bits(k, 64, 32, planes)
+        assert not bits(k, 64, 64, 300) and not bits(k, 40, 40, 300)
+    assert bits(7, 64, 64, 3000) and not bits(5, 64, 64, 3000)
