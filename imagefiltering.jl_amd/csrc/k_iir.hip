@@ -6,10 +6,13 @@
 // matrix M (Triggs & Sdika Eqs. 14-15), backward recursion and scaling.
 // Lines of up to 8192 elements run k_iir_line (contiguous axis, through an
 // LDS transpose) or k_iir_seg (strided axes): whole lines in registers, the
-// axis split into segments of one lane each.  Longer lines run k_iir_rows
-// (contiguous axis, LDS-staged chunks) or k_iir_strided (one thread per
-// line).  Lanes sit on adjacent lines, which are adjacent in memory for the
-// strided axes (coalesced).
+// axis split into segments of one lane each; short strided lines run
+// k_iir_short, one lane per line.  Longer lines run k_iir_rows (contiguous
+// axis, LDS-staged chunks) or k_iir_strided (one thread per line).  Lanes sit
+// on adjacent lines, which are adjacent in memory for the strided axes
+// (coalesced).
+#include <type_traits>
+
 #include "ifm_internal.h"
 
 namespace ifm {
@@ -661,19 +664,106 @@ __global__ void __launch_bounds__(64 * IS_MAXW) __attribute__((amdgpu_waves_per_
   else line_store<-1, LN>(p, g, tr, line0, w0, v);
 }
 
+// Strided lines of up to IK_MAX elements, one lane per line: no segments to
+// compose and, with S the next of a few lengths, few places of a lane's
+// registers unused.  The segmented form runs 64 elements for any of these
+// lines, and reads the 1- and 2-byte eltypes by a choice per element.  1 M lines
+// of 4 / 8 / 16 / 32 elements F64: 57 / 59 / 74 / 106 us segmented, 11 / 20 / 50 /
+// 101 this way; N0f8 -> F64 112 / 121 / 141 / 191 and 14 / 16 / 31 / 64.  Bound by
+// HBM from a million lines on.  Longer F32 and F64 lines fill segments well
+// enough (20000 of 40 F32: 6.3 us segmented, 7.2 this way); the smaller eltypes
+// gain up to 48 elements (1 M of 40 N0f8: 206 and 85).
+constexpr int IK_MAX = 32, IK_MAX_SMALL = 48;
+
+template <int DT, int S>
+__global__ void __launch_bounds__(256) k_iir_short(IirArgs p) {
+  const int64_t line = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (line >= p.lines) return;
+  const int n = p.n[p.axis], lead = S - n;  // v[lead ..]: the line
+  const int64_t base = (line % p.stride) + (line / p.stride) * p.stride * n;
+  using TE = decltype(line_ld<DT>(nullptr, 0));
+  constexpr int es = DT == IFM_F64 ? 8 : DT == IFM_F32 ? 4 : DT == IFM_U8 || DT == IFM_N0F8 ? 1 : 2;
+  TE x[S];
+  Walk q(p.src, base, p.stride, es);
+#pragma unroll
+  for (int j = 0; j < S; ++j) {  // every load unconditional, so that they are in flight together
+    x[j] = line_ld<DT>((const void *)q.at, 0);
+    q.next(j >= lead);
+  }
+  double v[S];
+#pragma unroll
+  for (int j = 0; j < S; ++j) v[j] = DT == IFM_N0F8 ? (double)x[j] / 255.0 : (double)x[j];
+  const double a1 = p.a[0], a2 = p.a[1], a3 = p.a[2];
+  const double b1 = p.b[0], b2 = p.b[1], b3 = p.b[2];
+  const double asum = a1 + a2 + a3, bsum = b1 + b2 + b3;
+  const double uminus = (p.isfill ? p.fill : v[0]) / (1 - asum);  // v[0]: the first element, or a copy of it
+  const double uplus = (p.isfill ? p.fill : v[S - 1]) / (1 - asum);
+  double y1 = uminus, y2 = uminus, y3 = uminus;
+#pragma unroll
+  for (int j = 0; j < S; ++j) {
+    if (j < lead) continue;  // uniform over the grid
+    v[j] = v[j] + a1 * y1 + a2 * y2 + a3 * y3;
+    y3 = y2;
+    y2 = y1;
+    y1 = v[j];
+  }
+  const double vplus = uplus / (1 - bsum);
+  const double d0 = y1 - uplus, d1 = y2 - uplus, d2 = y3 - uplus;
+  double z1 = p.M[0] * d0 + p.M[1] * d1 + p.M[2] * d2 + vplus;
+  double z2 = p.M[3] * d0 + p.M[4] * d1 + p.M[5] * d2 + vplus;  // beyond the edge
+  double z3 = p.M[6] * d0 + p.M[7] * d1 + p.M[8] * d2 + vplus;
+  v[S - 1] = z1;
+#pragma unroll
+  for (int j = S - 2; j >= 0; --j) {
+    if (j < lead) continue;
+    v[j] = v[j] + b1 * z1 + b2 * z2 + b3 * z3;
+    z3 = z2;
+    z2 = z1;
+    z1 = v[j];
+  }
+  const double sc = p.scale;
+  const auto store = [&](auto type) {
+    constexpr int DD = decltype(type)::value;
+    Walk w(p.dst, base, p.stride, DD == IFM_F64 ? 8 : DD == IFM_F32 ? 4 : 2);
+#pragma unroll
+    for (int j = 0; j < S; ++j) {
+      if (j < lead) continue;
+      iir_put<DD>(w.at, p.dt_dst, v[j] * sc);
+      w.next();
+    }
+  };
+  if (p.dt_dst == IFM_F64) store(std::integral_constant<int, IFM_F64>());
+  else if (p.dt_dst == IFM_F32) store(std::integral_constant<int, IFM_F32>());
+  else store(std::integral_constant<int, -1>());
+}
+
+template <int DT>
+static void short_go(const IirArgs &p, hipStream_t st) {
+  const int n = p.n[p.axis];
+  const dim3 grid((unsigned)((p.lines + 255) / 256)), blk(256);
+  if (n <= 8) hipLaunchKernelGGL((k_iir_short<DT, 8>), grid, blk, 0, st, p);
+  else if (n <= 16) hipLaunchKernelGGL((k_iir_short<DT, 16>), grid, blk, 0, st, p);
+  else if (n <= 32) hipLaunchKernelGGL((k_iir_short<DT, 32>), grid, blk, 0, st, p);
+  else hipLaunchKernelGGL((k_iir_short<DT, 48>), grid, blk, 0, st, p);
+}
+
 static int iir_waves(int n, int ln) { return (n + (64 / ln) * IS_S - 1) / ((64 / ln) * IS_S); }
 
 // Lines per workgroup: 32 (the longest runs of adjacent lines) when the
 // segments fit 8 waves, so that two workgroups share a CU, and there are
 // workgroups for every CU; fewer otherwise, but no fewer than 8 while the
 // segments fit 16 waves (200 x 150: 16.9 us with 8, 18.0 with 4; 3840 x 2160:
-// 71 with either).
-static int iir_lines(int n, int64_t lines) {
+// 71 with either), and no fewer than put the line into one wave, or a strided
+// one into three full ones (4000 strided lines F64, 64 / 128 / 192 elements:
+// 5.6 / 5.8 / 6.3 us, 7.3 / 7.5 / 7.8 with 8 lines and more elements before them).
+static int iir_lines(int n, int64_t lines, bool strided) {
   int ln = 32;
   while (ln > IS_MINL) {
     const int waves = iir_waves(n, ln);
     if (waves <= IS_MAXW / 2 && (lines + ln - 1) / ln >= 256) break;
     if (waves <= IS_MAXW && ln == 8) break;
+    if (waves == 1) break;
+    if (strided && waves == 3 && n % (64 / ln * IS_S) == 0) break;
     ln /= 2;
   }
   return ln;
@@ -695,7 +785,7 @@ static void seg_go(const IirArgs &p, const IirSegTables &tb, hipStream_t st) {
 
 template <int DT>
 static void seg_lines(const IirArgs &p, const IirSegTables &tb, hipStream_t st) {
-  switch (iir_lines(p.n[p.axis], p.lines)) {
+  switch (iir_lines(p.n[p.axis], p.lines, p.stride != 1)) {
   case 32: seg_go<DT, 32>(p, tb, st); break;
   case 16: seg_go<DT, 16>(p, tb, st); break;
   case 8: seg_go<DT, 8>(p, tb, st); break;
@@ -730,6 +820,17 @@ hipError_t launch_iir(const Dense4 &in, Dense4 &out, int axis, const IirCoef &c,
   p.isfill = isfill;
   p.fill = fill;
   if (p.lines == 0) return hipSuccess;
+  if (stride != 1 && in.n[axis] >= 4 && in.n[axis] <= (dtype_size(in.dtype) >= 4 ? IK_MAX : IK_MAX_SMALL)) {
+    switch (in.dtype) {
+    case IFM_F32: short_go<IFM_F32>(p, st); break;
+    case IFM_F64: short_go<IFM_F64>(p, st); break;
+    case IFM_BF16: short_go<IFM_BF16>(p, st); break;
+    case IFM_F16: short_go<IFM_F16>(p, st); break;
+    case IFM_N0F8: short_go<IFM_N0F8>(p, st); break;
+    default: short_go<IFM_U8>(p, st); break;
+    }
+    return hipGetLastError();
+  }
   if (iir_in_registers(in.n[axis])) {  // whole lines held in registers
     IirSegTables tb;
     // Built in extended precision and rounded once.

@@ -1125,6 +1125,47 @@ def test_iir_line_lengths(n, axis):
                 assert np.max(np.abs(got - want)) <= (tol + extra) * scale, (n, axis, border, T)
 
 
+@pytest.mark.parametrize("n", [4, 5, 8, 9, 15, 16, 17, 31, 32, 33, 47, 48, 49])
+def test_iir_short_strided_lines(n):
+    """Strided axes of a few elements, one lane per line: every register count's
+    edges, lines that do not fill the last workgroup, a middle axis and a last
+    one, every input and output eltype, in place.
+
+    Tolerance: as for the other lines (64 roundings at 2^-53 carried with weight
+    1 / (1 - sum a)); the output eltype adds its own rounding."""
+    rng = np.random.default_rng(n)
+    k = IF.KernelFactors.IIRGaussian(2.0)
+    tol = 64 * 2.0 ** -53 / (1 - k.asum)
+    for shape, axis in (((41, n, 9), 1), ((23, 12, n), 2)):
+        x64 = rng.standard_normal(shape)
+        codes = rng.integers(0, 256, shape).astype(np.uint8)
+        b16 = IF.bf16(x64)
+        cases = [(x64, x64), (x64.astype(np.float32), x64.astype(np.float32)), (x64.astype(np.float16), x64.astype(np.float16)),
+                 (IF.n0f8(codes), codes / 255.0), (codes, codes), (b16, IF.bf16_to_float32(b16))]
+        fac = (IF.KernelFactors.ReshapedOneD(3, axis, k),)
+        for a, ref in cases:
+            a = np.asfortranarray(a).view(type(a))
+            for border, ob in (("replicate", "replicate"), (IF.Fill(1.0), ("fill", 1.0))):
+                want = O.imfilter_iir(np.asfortranarray(np.asarray(ref, dtype=np.float64)),
+                                      [(axis, k.a, k.b, k.scale, k.M)], ob)
+                scale = np.max(np.abs(want))
+                for T, extra in ((IF.Float64, 0.0), (IF.Float32, 2.0 ** -24), (IF.Float16, 2.0 ** -11), (IF.BFloat16, 2.0 ** -8)):
+                    got = IF.imfilter(T, a, fac, border, IF.Algorithm.IIR())
+                    got = np.asarray(IF.bf16_to_float32(got) if T is IF.BFloat16 else got, dtype=np.float64)
+                    assert np.max(np.abs(got - want)) <= (tol + extra) * scale, (n, axis, border, T)
+        d = IF.DeviceArray.from_host(np.asfortranarray(x64))
+        want = IF.imfilter(IF.Float64, d, fac, "replicate", IF.Algorithm.IIR()).to_host()
+        from imagefiltering import _lib
+        from imagefiltering.device import ifm_array
+        from imagefiltering.imfilter import _border_struct
+        f = (_lib.IfmIir * 1)()
+        f[0].axis, f[0].scale = axis, k.scale
+        f[0].a[:], f[0].b[:], f[0].M[:] = list(k.a), list(k.b), [float(m) for m in np.asarray(k.M).ravel()]
+        _lib.check(_lib.load().ifm_imfilter_iir(_lib.ctx(), ifm_array(d), ifm_array(d), f, 1,
+                                                _border_struct(IF.borderinstance("replicate"), IF.Float64)))
+        np.testing.assert_array_equal(d.to_host(), want)
+
+
 @pytest.mark.parametrize("sigma", [5.0, 10.0, 20.0])
 @pytest.mark.parametrize("n", [200, 513, 1000, 4097])
 @pytest.mark.parametrize("axis", [0, 1])
