@@ -9,7 +9,9 @@ workgroups, which counts when an image has too few tiles to fill the 256
 compute units.  Which wins depends on the kernel length, the image size and
 the input type, so `tune` times both shapes on synthetic images for every
 (input dtype, kernel-length bucket, image-size bucket), keeps the faster and
-installs the result as rules.  `save` / `load` keep them as JSON, and the
+installs the result as rules.  Large images with factors of equal length take
+no tiles at all (they are marched down in strips), so the trials run pairs of
+unequal length, which always do.  `save` / `load` keep them as JSON, and the
 process-wide context installs the cached rules when it is created, so a
 machine tunes once.  Results do not depend on the tile shape: every output
 sums the same taps in the same order.
@@ -31,6 +33,8 @@ KBUCKETS = ((9, 7), (17, 13), (33, 29), (64, 49))
 # (max output pixels, representative side): square images of that side.
 SIZEBUCKETS = ((384 ** 2, 256), (1536 ** 2, 1024), (3072 ** 2, 2048), (1 << 62, 4096))
 DTYPES = ("Float32", "BFloat16")
+# Of a saved result with trials; the first trials (no format) ran equal pairs.
+FORMAT = 2
 _DT_CODE = {"Float32": 2, "Float64": 3, "BFloat16": 4, "Float16": 5, "N0f8": 1, "UInt8": 0}
 
 
@@ -88,13 +92,15 @@ def save(result, path=None):
 def load(path=None):
     """Install the rules of a saved tuning result; returns it (None if there
     is no cache file, or if it cannot be read: the default tiles then stay,
-    with a warning)."""
+    with a warning).  Rules of trials that did not time the tiles are not used."""
     path = path or cache_path()
     if not os.path.exists(path):
         return None
     try:
         with open(path) as f:
             result = json.load(f)
+        if "trials" in result and result.get("format") != FORMAT:
+            raise ValueError("its trials are of another format: tune again")
         install(result["rules"])
     except Exception as e:  # a stale or damaged cache must not break filtering
         import warnings
@@ -104,21 +110,22 @@ def load(path=None):
 
 
 def _factors(k):
-    """A normalised box pair of k taps each, centred (the taps' values do not
+    """A normalised box pair of k and k - 2 taps, centred (the taps' values do not
     change the kernel's time)."""
-    t = np.full(k, 1.0 / k)
-    fa = (_lib.IfmFactor * 2)()
-    for axis in range(2):
-        fa[axis].axis, fa[axis].len, fa[axis].first = axis, k, -(k // 2)
+    fa, keep = (_lib.IfmFactor * 2)(), []
+    for axis, n in ((0, k), (1, k - 2)):
+        t = np.full(n, 1.0 / n)
+        fa[axis].axis, fa[axis].len, fa[axis].first = axis, n, -(n // 2)
         fa[axis].taps = t.ctypes.data_as(C.POINTER(C.c_double))
-    return fa, t
+        keep.append(t)
+    return fa, keep
 
 
 def tune(dtypes=DTYPES, kbuckets=KBUCKETS, sizebuckets=SIZEBUCKETS, rounds=3, target_ms=4.0):
     """Time every tile height on every bucket; install and return
-    {"rules": [...], "trials": [...]}.  Each trial runs the fused kernel on a
-    square image of the bucket's side with a kernel of the bucket's length,
-    'reflect' border, F64 output (the eltype imfilter gives F32 or BF16 pixels
+    {"format": FORMAT, "rules": [...], "trials": [...]}.  Each trial runs the fused
+    kernel on a square image of the bucket's side with a pair whose longer factor
+    has the bucket's length, 'reflect' border, F64 output (the eltype imfilter gives F32 or BF16 pixels
     with F64 taps); the time per call is the best of `rounds` runs of enough
     calls to fill about target_ms."""
     from .device import DeviceArray, ifm_array
@@ -157,7 +164,7 @@ def tune(dtypes=DTYPES, kbuckets=KBUCKETS, sizebuckets=SIZEBUCKETS, rounds=3, ta
                             _lib.check(L.ifm_timer_stop(ctx, C.byref(ms)))
                             t.append(ms.value / reps)
                         best[th] = min(t)
-                        trials.append({"dtype": dt, "side": side, "k": k, "tile_h": th, "us": round(best[th] * 1e3, 3)})
+                        trials.append({"dtype": dt, "side": side, "k": [k, k - 2], "tile_h": th, "us": round(best[th] * 1e3, 3)})
                     choices[(dt, kmax, maxpx)] = min(best, key=best.get)
                     del keep
                 del img, out
@@ -166,7 +173,7 @@ def tune(dtypes=DTYPES, kbuckets=KBUCKETS, sizebuckets=SIZEBUCKETS, rounds=3, ta
         raise
     rules = rules_from_choices(choices)
     install(rules)
-    return {"rules": rules, "trials": trials}
+    return {"format": FORMAT, "rules": rules, "trials": trials}
 
 
 if __name__ == "__main__":

@@ -129,3 +129,33 @@ def test_damaged_cache_is_ignored(tmp_path, monkeypatch):
     assert tiles.load(str(p))["rules"][0]["tile_h"] == 64
     assert installed and installed[-1][0]["kmax"] == 9
     assert tiles.load(str(tmp_path / "absent.json")) is None
+
+
+def test_trials_run_pairs_that_take_tiles():
+    """Every pair the tuner times is one that no image size marches, with the
+    bucket's length as its longer factor."""
+    marched = _lib.load()._ZN3ifm17sep_march_batchedEiiilll
+    marched.argtypes, marched.restype = [C.c_int] * 3 + [C.c_int64] * 3, C.c_bool
+    for kmax, k in tiles.KBUCKETS:
+        fa, keep = tiles._factors(k)
+        k0, k1 = fa[0].len, fa[1].len
+        assert max(k0, k1) == k and (fa[0].axis, fa[1].axis) == (0, 1)
+        assert k0 != k1  # the marched kernel exists for equal pairs only
+        for dt in range(6):
+            assert not marched(k0, k1, dt, 4096, 4096, 1 << 40)
+        for f, t in zip(fa, keep):
+            assert f.first == -(f.len // 2) and abs(sum(f.taps[: f.len]) - 1) < 1e-12 and len(t) == f.len
+
+
+def test_rules_of_other_trials_are_ignored(tmp_path, monkeypatch):
+    p = tmp_path / "tiles.json"
+    rule = {"op": 1, "dtype": 2, "kmax": 17, "tile_h": 64, "max_pixels": 1 << 62}
+    trial = {"dtype": "Float32", "side": 4096, "k": 13, "tile_h": 64, "us": 39.9}
+    installed = []
+    monkeypatch.setattr(tiles, "install", lambda rules: installed.append(rules))
+    tiles.save({"rules": [rule], "trials": [trial]}, str(p))
+    with pytest.warns(UserWarning):
+        assert tiles.load(str(p)) is None
+    assert not installed
+    tiles.save({"format": tiles.FORMAT, "rules": [rule], "trials": [dict(trial, k=[13, 11])]}, str(p))
+    assert tiles.load(str(p))["rules"] == [rule] and installed == [[rule]]
