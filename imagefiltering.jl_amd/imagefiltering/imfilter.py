@@ -7,6 +7,9 @@ choice (filter_algorithm) and resource.  Every algorithm then runs on the GPU
 through libifm; there is no CPU compute path.  Julia's `imfilter!` is
 `imfilter_` here.
 """
+import math
+import sys
+
 import numpy as np
 
 from . import _lib
@@ -115,19 +118,24 @@ def factorkernel(kernel):
     return (OffsetArray(u, (k.first[0], 0)), OffsetArray(v, (0, k.first[1])))
 
 
+_RANK_EPS = math.sqrt(sys.float_info.epsilon)
+
+
 def _far_from_rank_one(a):
-    """Whether some S[i], i >= 1, is certainly at least eps = sqrt(2^-52), without
-    the SVD (21 x 21: a tenth of its time).  If all were smaller, a = B + E with B
-    of rank one and |E| < eps elementwise; then, with p = a[i, j] the largest
-    entry, |a[k, l] - a[k, j] a[i, l] / p| <= 4 eps + 6 eps^2 / p, which is below
-    16 eps for p >= eps, rounding (a few 2^-53 p) left out."""
-    eps = np.sqrt(np.finfo(np.float64).eps)
-    i, j = divmod(int(np.abs(a).argmax()), a.shape[1])
-    p = a[i, j]
-    if not abs(p) >= eps:
-        return False
-    r = a - a[:, j:j + 1] * (a[i] / p)
-    return bool(max(r.max(), -r.min()) > 16 * eps + 1e-14 * abs(p))
+    """Whether S[1] is certainly at least eps = sqrt(2^-52), without the SVD.  The
+    smaller singular value of a 2 x 2 submatrix X is no larger than S[1], and at
+    least |det X| / |X|; the SVD's own S[1] is off by a few times 2^-53 |a|.  Three
+    submatrices tell most kernels apart and cost a rank-one kernel 2 us of the 20
+    to 50 that its SVD takes; entries that are not finite leave it to the SVD."""
+    m, n = a.shape
+    for i, j, k, l in ((m // 4, n // 4, m // 2, n // 2), (0, 0, m // 2, n // 2), (m // 2, n // 3, m - 1, n - 1)):
+        p, q, r, s = a.item(i, j), a.item(i, l), a.item(k, j), a.item(k, l)
+        x, y = p * s, q * r
+        size = abs(p) + abs(q) + abs(r) + abs(s)
+        if abs(x - y) > 2 * _RANK_EPS * size + 1e-15 * (abs(x) + abs(y)):
+            if abs(x - y) > (2 * _RANK_EPS + 1e-13 * math.sqrt(np.vdot(a, a))) * size:
+                return True
+    return False
 
 
 def _kernel_dtype(k):

@@ -320,3 +320,26 @@ def test_median_bit_plane_rule():
             assert not bits(k, 24, 24, planes) and not bits(k, 64, 32, planes)
         assert not bits(k, 64, 64, 300) and not bits(k, 40, 40, 300)
     assert bits(7, 64, 64, 3000) and not bits(5, 64, 64, 3000)
+
+
+def test_factorkernel_common_kernels(monkeypatch):
+    """Kernels in common use that are not of rank one are told apart without the
+    SVD; rank-one ones, thin ones and ones with entries that are not finite are
+    left to it, whatever their scale."""
+    import sys
+    m = sys.modules["imagefiltering.imfilter"]
+    rng = np.random.default_rng(4)
+    y, x = np.mgrid[-5:6, -5:6]
+    far = [np.asarray(k.data) for k in (IF.Kernel.LoG(2.0), IF.Kernel.LoG(8.0), IF.Kernel.DoG(2.0))]
+    far += [rng.standard_normal((n, n + d)) for n in (2, 3, 7, 21, 45) for d in (0, 1)]
+    far += [np.array([[0, 1, 0], [1, -4, 1], [0, 1, 0.0]]), (np.hypot(x, y) <= 5) * 1.0, np.eye(9), np.asfortranarray(rng.random((6, 4)))]
+    near = [np.outer(rng.standard_normal(a), rng.standard_normal(b)) * s for a, b in ((2, 2), (3, 5), (7, 7), (21, 21))
+            for s in (1e-12, 1e-3, 1.0, 1e9)]
+    near += [rng.random((1, 7)), rng.random((7, 1)), np.zeros((5, 5)), np.full((7, 7), np.nan), np.full((4, 4), np.inf)]
+    with np.errstate(all="raise"):
+        assert not any(m._far_from_rank_one(a) for a in near)
+        assert all(m._far_from_rank_one(a) for a in far)
+    monkeypatch.setattr(np.linalg, "svd", None)
+    for a in far:
+        k, = IF.factorkernel(IF.centered(a))
+        np.testing.assert_array_equal(np.asarray(k.data), a)
