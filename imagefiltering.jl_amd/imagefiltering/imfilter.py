@@ -606,9 +606,11 @@ def _choose(r, alg, img, kernel):
 
 def _run_default(out, img, kernel, border):
     """filter_algorithm's choice for one long dense kernel on a device array,
-    made on the device (ifm_imfilter_default); False where the host decides."""
+    made on the device (ifm_imfilter_default); False where the host decides
+    (Float64 pixels always: asking the library first cost those calls 10 us)."""
     if not (len(kernel) == 1 and isinstance(kernel[0], OffsetArray) and isinstance(border, (Pad, Fill))
-            and isinstance(img, DeviceArray) and img.eltype.kind == "float" and maxlen(kernel) > 30):
+            and isinstance(img, DeviceArray) and img.eltype.kind == "float" and img.eltype is not Float64
+            and maxlen(kernel) > 30):
         return False
     comps = _components(kernel, len(img.shape))
     if len(comps) != 1 or comps[0].kind != "dense":

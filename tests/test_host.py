@@ -343,3 +343,13 @@ def test_factorkernel_common_kernels(monkeypatch):
     for a in far:
         k, = IF.factorkernel(IF.centered(a))
         np.testing.assert_array_equal(np.asarray(k.data), a)
+
+
+def test_default_algorithm_of_float64_images_is_the_hosts():
+    """No library call is made to learn that Float64 pixels are not taken."""
+    import sys
+    m = sys.modules["imagefiltering.imfilter"]
+    img = object.__new__(IF.DeviceArray)
+    img.shape, img.eltype, img.order, img._ptr = (100, 90), IF.Float64, "F", None
+    kern = (IF.centered(np.random.default_rng(0).random((9, 9))),)
+    assert m._run_default(None, img, kern, IF.borderinstance("reflect")) is False
