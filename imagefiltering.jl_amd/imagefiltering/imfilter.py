@@ -91,6 +91,9 @@ def _as_offset(k):
     return OffsetArray(a, (1,) * a.ndim)   # a plain array inside a tuple keeps its 1-based axes
 
 
+_RANK_EPS = math.sqrt(sys.float_info.epsilon)
+
+
 def factorkernel(kernel):
     """src/imfilter.jl:1156-1184: a 2-D kernel is tested for rank 1 with
     svd (tolerance sqrt(eps)); rank 1 -> two factors scaled by sqrt(s)."""
@@ -107,18 +110,14 @@ def factorkernel(kernel):
         data = data.astype(np.float64)
     if data.dtype == np.float64 and data.size and _far_from_rank_one(data):
         return (k,)
-    U, S, Vt = np.linalg.svd(data.astype(np.float64) if data.dtype != np.float32 else data)
-    eps = np.sqrt(np.finfo(S.dtype).eps)
-    separable = all(abs(S[i]) < eps for i in range(1, len(S)))
-    if not separable:
+    U, S, Vt = np.linalg.svd(data.astype(np.float64, copy=False) if data.dtype != np.float32 else data)
+    eps = _RANK_EPS if S.dtype == np.float64 else np.sqrt(np.finfo(S.dtype).eps)
+    if len(S) > 1 and not S[1] < eps:  # in descending order
         return (k,)   # the reference's leading dummykernel is a copy and is skipped
     ss = np.sqrt(S[0])
-    u = (ss * U[:, 0:1]).astype(data.dtype)
-    v = (ss * Vt[0:1, :]).astype(data.dtype)
+    u = (ss * U[:, 0:1]).astype(data.dtype, copy=False)
+    v = (ss * Vt[0:1, :]).astype(data.dtype, copy=False)
     return (OffsetArray(u, (k.first[0], 0)), OffsetArray(v, (0, k.first[1])))
-
-
-_RANK_EPS = math.sqrt(sys.float_info.epsilon)
 
 
 def _far_from_rank_one(a):
