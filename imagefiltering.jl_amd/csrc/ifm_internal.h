@@ -392,10 +392,13 @@ struct SepReq {
   int ty;  // tile height (S2_TY or S2_TY2), or rows per chunk of a marched request
 };
 // Whether an image is marched (sep_march) with equal factors of a length that
-// can be, whether a request of n0 x n1 is in a batch of so many pixels, and the
-// workgroups and rows per chunk of a marched request.
+// can be.
 bool sep_march_pays(int k, int dt_in, int64_t o0, int64_t o1, int64_t nplanes);
-bool sep_march_batched(int k0, int k1, int dt_in, int64_t n0, int64_t n1, int64_t batch_pixels);
+// In a batch: whether its pixels are enough for a length, what a request's own
+// shape and eltypes say, and the workgroups and rows per chunk of a marched one.
+enum { SM_NEVER = 0, SM_SLOWER = 1, SM_FASTER = 2 };
+bool sep_march_line(int k, int64_t batch_pixels);
+int sep_march_shape(int k0, int k1, int dt_in, int dt_out, int64_t n0, int64_t n1);
 int sep_march_groups(int n0, int n1, int *rows);
 hipError_t launch_sep_march_batch(const SepReq *reqs, const int *tile_req, const int *tile_first, int ntiles,
                                   hipStream_t st);

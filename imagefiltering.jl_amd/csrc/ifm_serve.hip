@@ -236,12 +236,25 @@ int build_batch(ifm_ctx *ctx, const ifm_request *reqs, const int *idx, int n, co
                 std::vector<Group> &groups, Extra &ex) {
   std::vector<int> &fallback = ex.alone, &band = ex.band;
   std::vector<Dense4> vin(n), vout(n);
-  int64_t sep_pixels = 0;  // of the separable requests
+  int64_t sep_pixels = 0, faster_pixels = 0, slower_pixels = 0;  // of the separable requests; by what marching does to them
+  std::vector<char> shape(2 * (size_t)n);
   for (int i = 0; i < n; ++i) {
     const ifm_request &q = reqs[idx[i]];
     int rc = check_request(ctx, q, vin[i], vout[i]);
     if (rc) return rc;
-    if (q.op == IFM_OP_SEPARABLE) sep_pixels += vin[i].n[0] * vin[i].n[1] * (q.nfactors2 > 0 ? 2 : 1);
+    if (q.op != IFM_OP_SEPARABLE) continue;
+    const int64_t pixels = vin[i].n[0] * vin[i].n[1];
+    for (int part = 0; part < (q.nfactors2 > 0 ? 2 : 1); ++part) {
+      const int nf = part ? q.nfactors2 : q.nfactors;
+      const ifm_factor *fs = part ? q.factors2 : q.factors;
+      int k[2] = {1, 1};
+      for (int f = 0; f < nf; ++f) k[fs[f].axis] = fs[f].len;
+      const int s = sep_march_shape(k[0], k[1], vin[i].dtype, part ? q.out2.dtype : vout[i].dtype, vin[i].n[0], vin[i].n[1]);
+      shape[2 * (size_t)i + part] = (char)s;
+      sep_pixels += pixels;
+      if (s == SM_FASTER) faster_pixels += pixels;
+      if (s == SM_SLOWER) slower_pixels += pixels;
+    }
   }
   auto tiles_group = [&](int kind, int param, const std::vector<int> &members, const std::vector<int> &ntile,
                          size_t reqs_off, size_t lds) {
@@ -277,7 +290,7 @@ int build_batch(ifm_ctx *ctx, const ifm_request *reqs, const int *idx, int n, co
   }
   // Separable: the ones in tiles and the marched requests, in one pass over the
   // requests (4000 of 64 x 64: 142 us on the host before there were two groups,
-  // 183 with a pass for each and one for the pixels, 155 this way).
+  // 183 with a pass for each and one for the pixels, 153 this way).
   struct {
     std::vector<int> mem, nt;
     std::vector<SepReq> sr;
@@ -318,7 +331,12 @@ int build_batch(ifm_ctx *ctx, const ifm_request *reqs, const int *idx, int n, co
       s.dt_in = vin[i].dtype;
       s.dt_out = part ? q.out2.dtype : vout[i].dtype;
       s.fill = (float)q.border.fill;
-      const bool marched = sep_march_batched(k0, k1, s.dt_in, s.n0, s.n1, sep_pixels);
+      // a few slower requests go along with the others: a launch of their own
+      // costs more (the serving mix, 512 requests a batch: 121,000 images/s all
+      // marched, 118,000 with its narrow images in tiles)
+      const int how = shape[2 * (size_t)i + part];
+      const bool marched = (how == SM_FASTER || (how == SM_SLOWER && 4 * slower_pixels <= faster_pixels)) &&
+                           sep_march_line(k0, sep_pixels);
       auto &g = sep[marched];
       if (g.sr.empty()) {
         g.sr.reserve(n);

@@ -386,9 +386,9 @@ bool sep_march_pays(int k, int dt_in, int64_t o0, int64_t o1, int64_t nplanes) {
 }
 
 static bool sep_march_takes(int k0, int k1, int dt_in) {
-  const bool k = k0 == 3 || k0 == 5 || k0 == 7 || k0 == 9 || k0 == 13 || k0 == 17 || k0 == 21 || k0 == 25 || k0 == 29 ||
-                 k0 == 33;
-  return k0 == k1 && k && dt_in != IFM_F64;
+  constexpr uint64_t lengths = 1ull << 3 | 1ull << 5 | 1ull << 7 | 1ull << 9 | 1ull << 13 | 1ull << 17 | 1ull << 21 |
+                               1ull << 25 | 1ull << 29 | 1ull << 33;
+  return k0 == k1 && k0 < 64 && (lengths >> k0 & 1) && dt_in != IFM_F64;
 }
 
 static bool march_launch(const Sep2dArgs &s, hipStream_t st) {
@@ -738,15 +738,19 @@ __global__ void __launch_bounds__(256) k_sep_march_batch(const SepReq *__restric
 // longest factors) and end with its longest waves, so the line is drawn higher
 // than for one image.  Batches of the serving mix (sides up to 2048), in tiles
 // and marched: 24 requests 143 / 172 us, 48: 231 / 246, 96: 441 / 393, 256: 830
-// / 715.  Above it the request's own shape and eltype decide, as for one image:
-// 1000 of 60 x 300, 9 taps: F32 95 / 135, bf16 81 / 171; 300 of 300 x 200: 101 /
-// 102 and 81 / 121; 200 of 512 x 200: 100 / 88 and 83 / 95.
+// / 715.  Above it the request's own shape and eltypes decide, as for one image
+// (247 batches of equal requests): 1000 of 60 x 300, 9 taps: F32 95 / 135, bf16
+// to bf16 81 / 171; 300 of 300 x 200: 101 / 102 and 81 / 121; 200 of 512 x 200:
+// 100 / 88 and 83 / 95.  16-bit pixels with wider results gain more than with
+// 16-bit ones: 59 of 2048 x 2048, 33 taps bf16 to F64 2071 / 1668.
 constexpr int SM_BATCH_ROWS = 32;  // rows per chunk
-bool sep_march_batched(int k0, int k1, int dt_in, int64_t n0, int64_t n1, int64_t batch_pixels) {
-  if (!sep_march_takes(k0, k1, dt_in) || batch_pixels * 13 < SM_BATCH_PIXELS * std::max(k0, 13)) return false;
-  const double speed = k0 <= 9 ? 1.27 : k0 < 21 ? 1.3 : 1.5;
+bool sep_march_line(int k, int64_t batch_pixels) { return batch_pixels * 13 >= SM_BATCH_PIXELS * std::max(k, 13); }
+int sep_march_shape(int k0, int k1, int dt_in, int dt_out, int64_t n0, int64_t n1) {
+  if (!sep_march_takes(k0, k1, dt_in)) return SM_NEVER;
+  if (n0 <= S2_TX) return SM_SLOWER;  // a strip half empty at least
+  const double speed = k0 < 21 ? 1.3 : 1.5, wide = dt_out == IFM_F32 || dt_out == IFM_F64 ? 0.78 : 0.66;
   const MarchFill f(k0, n0, n1, SM_BATCH_ROWS);
-  return speed * march_eltype(dt_in, 0.8, 0.7) * f.columns * f.tiled >= f.cover * f.marched;
+  return speed * march_eltype(dt_in, 0.75, wide) * f.columns * f.tiled >= f.cover * f.marched ? SM_FASTER : SM_SLOWER;
 }
 
 // Workgroups of a marched request, and its rows per chunk.

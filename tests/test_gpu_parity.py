@@ -1429,14 +1429,15 @@ def _separable_request(shape, et, oet, k, border, seed, k1=None, second=False):
 
 def test_marched_batch_equals_requests_alone():
     """A batch above the marching line, with every marched length, requests that
-    stay in tiles beside them (other lengths, narrow images, 16-bit pixels),
-    small ones whose strips and chunks are ragged, two outputs, every border: bit
-    for bit the same requests run alone, below the line."""
+    stay in tiles beside them (other lengths), a few that go along (narrow images,
+    16-bit pixels), small ones whose strips and chunks are ragged, two outputs,
+    every border: bit for bit the same requests run alone, below the line."""
     import ctypes as C
     from imagefiltering import _lib
     L, ctx = _lib.load(), _lib.ctx()
-    marched = L._ZN3ifm17sep_march_batchedEiiilll
-    marched.argtypes, marched.restype = [C.c_int] * 3 + [C.c_int64] * 3, C.c_bool
+    shape_of, line = L._ZN3ifm15sep_march_shapeEiiiill, L._ZN3ifm14sep_march_lineEil
+    shape_of.argtypes, shape_of.restype = [C.c_int] * 4 + [C.c_int64] * 2, C.c_int
+    line.argtypes, line.restype = [C.c_int, C.c_int64], C.c_bool
     borders = STYLES + [IF.Fill(0.25)]
     specs = []  # shape, eltype, output eltype, lengths, two outputs
     for i, k in enumerate((3, 5, 7, 9, 13, 17, 21, 25, 29, 33)):
@@ -1447,8 +1448,11 @@ def test_marched_batch_equals_requests_alone():
               ((300, 200), IF.Float32, IF.Float32, 11, 11, False), ((300, 200), IF.Float32, IF.Float64, 9, 13, True),
               ((1, 1), IF.Float32, IF.Float32, 3, 3, False)]
     px = sum(s[0] * s[1] * (2 if two else 1) for s, *_, two in specs)
-    took = [marched(k0, k1, et.code, *shape, px) for shape, et, _, k0, k1, _ in specs]
-    assert sum(took) >= 20 and not all(took)
+    how = [shape_of(k0, k1, et.code, oet.code, *shape) for shape, et, oet, k0, k1, _ in specs]
+    sizes = [s[0] * s[1] * (2 if two else 1) for s, *_, two in specs]
+    faster, slower = (sum(n for n, h in zip(sizes, how) if h == m) for m in (2, 1))
+    took = [h > (1 if 4 * slower > faster else 0) and line(s[3], px) for s, h in zip(specs, how)]
+    assert sum(took) >= 20 and not all(took) and set(how) == {0, 1, 2}
     assert {s[3] for s, m in zip(specs, took) if m and s[1] is IF.Float32 and s[0][0] == 421} >= {3, 5, 7, 9, 13, 17, 21}
     reqs, outs, keep = [], [], []
     for i, (shape, et, oet, k0, k1, two) in enumerate(specs):
@@ -1458,7 +1462,7 @@ def test_marched_batch_equals_requests_alone():
         outs.append(o)
         keep.append(x)
         one = (_lib.IfmRequest * 1)(q)
-        assert not marched(k0, k1, et.code, *shape, shape[0] * shape[1] * (2 if two else 1))
+        assert not line(k0, shape[0] * shape[1] * (2 if two else 1))
         _lib.check(L.ifm_batch_run(ctx, one, 1))
     _lib.check(L.ifm_ctx_synchronize(ctx))
     alone = [[d.to_host() for d in o] for o in outs]

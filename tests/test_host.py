@@ -287,20 +287,22 @@ def test_separable_march_rule():
 def test_separable_march_rule_of_batches():
     import ctypes as C
     from imagefiltering import _lib
-    marched = _lib.load()._ZN3ifm17sep_march_batchedEiiilll
-    marched.argtypes, marched.restype = [C.c_int] * 3 + [C.c_int64] * 3, C.c_bool
-    big = 1 << 28
+    L = _lib.load()
+    shape, line = L._ZN3ifm15sep_march_shapeEiiiill, L._ZN3ifm14sep_march_lineEil
+    shape.argtypes, shape.restype = [C.c_int] * 4 + [C.c_int64] * 2, C.c_int
+    line.argtypes, line.restype = [C.c_int, C.c_int64], C.c_bool
+    NEVER, SLOWER, FASTER = range(3)
     for k in (3, 5, 7, 9, 13, 17, 21, 25, 29, 33):
-        line = 16_000_000 * max(k, 13) // 13
-        assert not marched(k, k, F32, 1024, 1024, line - 1)
-        assert marched(k, k, F32, 1024, 1024, line + 1)
-        assert not marched(k, k, F64, 1024, 1024, big)
-        assert not marched(k, k + 2, F32, 1024, 1024, big)
+        px = 16_000_000 * max(k, 13) // 13
+        assert not line(k, px - 1) and line(k, px + 1)
+        assert shape(k, k, F32, F64, 1024, 1024) == FASTER and shape(k, k, BF16, F64, 1024, 1024) == FASTER
+        assert shape(k, k, F64, F64, 1024, 1024) == shape(k, k + 2, F32, F64, 1024, 1024) == NEVER
         for dt in (N0F8, F32, BF16):
-            assert not marched(k, k, dt, 60, 300, big)
-            assert not marched(k, k, dt, 64, 64, big)
-        assert marched(k, k, BF16, 1024, 1024, big) == (k >= 21)
-    assert not marched(11, 11, F32, 1024, 1024, big)
+            assert shape(k, k, dt, F64, 60, 300) == shape(k, k, dt, F32, 64, 64) == SLOWER
+        assert shape(k, k, BF16, BF16, 300, 64) == SLOWER
+        if k < 21:
+            assert shape(k, k, BF16, BF16, 1000, 1000) == SLOWER
+    assert shape(11, 11, F32, F64, 1024, 1024) == NEVER
 
 
 def test_median_bit_plane_rule():

@@ -134,15 +134,15 @@ def test_damaged_cache_is_ignored(tmp_path, monkeypatch):
 def test_trials_run_pairs_that_take_tiles():
     """Every pair the tuner times is one that no image size marches, with the
     bucket's length as its longer factor."""
-    marched = _lib.load()._ZN3ifm17sep_march_batchedEiiilll
-    marched.argtypes, marched.restype = [C.c_int] * 3 + [C.c_int64] * 3, C.c_bool
+    shape = _lib.load()._ZN3ifm15sep_march_shapeEiiiill
+    shape.argtypes, shape.restype = [C.c_int] * 4 + [C.c_int64] * 2, C.c_int
     for kmax, k in tiles.KBUCKETS:
         fa, keep = tiles._factors(k)
         k0, k1 = fa[0].len, fa[1].len
         assert max(k0, k1) == k and (fa[0].axis, fa[1].axis) == (0, 1)
         assert k0 != k1  # the marched kernel exists for equal pairs only
         for dt in range(6):
-            assert not marched(k0, k1, dt, 4096, 4096, 1 << 40)
+            assert shape(k0, k1, dt, dt, 4096, 4096) == 0
         for f, t in zip(fa, keep):
             assert f.first == -(f.len // 2) and abs(sum(f.taps[: f.len]) - 1) < 1e-12 and len(t) == f.len
 
