@@ -1242,8 +1242,9 @@ def test_iir_in_and_out_share_memory(n, ein, eout, shift):
 @pytest.mark.parametrize("shape", [(9, 9), (31, 64), (127, 63), (128, 65), (129, 64), (163, 130), (288, 33)])
 def test_median_codes_tile_edges(k, shape):
     """Tile and word edges of the bit-plane median (128 x 64 tiles, words of 32
-    columns) on enough planes for it to be taken (192 tiles), every border,
-    code and Float32 results, an Inner() interior: bit-exact."""
+    columns) on 192 tiles, every border, code and Float32 results, an Inner()
+    interior: bit-exact.  (5 x 5 and 7 x 7 windows take the network on the smaller
+    of these planes; the stacks of the next test take bit planes.)"""
     from imagefiltering import _lib
     from imagefiltering.device import ifm_array
     rng = np.random.default_rng(k * 1000 + shape[0])
@@ -1343,8 +1344,8 @@ def test_median_float64_networks(k, shape):
 @pytest.mark.parametrize("shape", [(128, 35), (131, 70), (255, 17)])
 def test_fir_march_equals_tiles(k, shape):
     """The marched form sums every output in the tiles' order: a stack of planes
-    large enough to be marched equals its planes filtered alone (too small to
-    be), bit for bit, over eltypes, borders, ragged strips and chunks, and an
+    of the size that is marched (where the eltype gains by it) equals its planes
+    filtered alone (too small to be), bit for bit, over eltypes, borders, ragged strips and chunks, and an
     output region that starts inside the image."""
     rng = np.random.default_rng(k + shape[0])
     taps = [rng.standard_normal(k), rng.standard_normal(k)]
