@@ -1345,8 +1345,8 @@ def test_median_float64_networks(k, shape):
 def test_fir_march_equals_tiles(k, shape):
     """The marched form sums every output in the tiles' order: a stack of planes
     of the size that is marched (where the eltype gains by it) equals its planes
-    filtered alone (too small to be), bit for bit, over eltypes, borders, ragged strips and chunks, and an
-    output region that starts inside the image."""
+    filtered alone (too small to be), bit for bit, over eltypes, borders, ragged
+    strips and chunks, and an output region that starts inside the image."""
     rng = np.random.default_rng(k + shape[0])
     taps = [rng.standard_normal(k), rng.standard_normal(k)]
     planes = -(-4_000_000 * max(k, 13) // 13 // ((shape[0] - 2) * (shape[1] - 2))) + 1
