@@ -349,9 +349,9 @@ static int march_rows(int64_t o1, int64_t strips, int k) {
 constexpr int64_t SM_PIXELS = 4000000, SM_BATCH_PIXELS = 16000000;
 
 // Above that line the speed over tiles is estimated from what it was measured
-// to depend on (816 shapes: 20 to 4096 columns in one plane and in stacks, 3 to
-// 33 taps, F32, bf16 and N0f8, 1 to 3 times the line; what marches by this rule
-// was at worst 0.93 of the tiles' speed, and 0.53 before there was one):
+// to depend on (1206 shapes: 20 to 4096 columns in one plane and in stacks, 3 to
+// 33 taps, F32, 16-bit floats and N0f8, 1 to 4 times the line; what marches by
+// this rule was at worst 0.92 of the tiles' speed, and 0.53 before there was one):
 //  * columns: the filled part of 128-column strips against that of 64-column
 //    tiles.  13 taps, N0f8: 60 x 90000 24.7 us in tiles, 33.2 marched; 4096 wide
 //    and as large 26.3 and 26.6.
@@ -362,6 +362,8 @@ constexpr int64_t SM_PIXELS = 4000000, SM_BATCH_PIXELS = 16000000;
 //    at three times that.
 //  * eltype: single elements of 1 and 2 bytes are loaded where F32 comes in
 //    pairs.  21 taps bf16: 0.85 at the line, 1.10 at three times that.
+// Where the line lies matters to both sides: 29 taps bf16 to F64 on 4096^2, at
+// 1.9 times the line, 115 us in tiles and 93 marched.
 struct MarchFill {
   double columns, cover;  // 64-column tiles and the half strips over them
   double tiled, marched;  // rows of the tiles, and of chunks with what precedes them over that of a full chunk
@@ -380,9 +382,10 @@ bool sep_march_pays(int k, int dt_in, int64_t o0, int64_t o1, int64_t nplanes) {
   const double line = (double)SM_PIXELS * std::max(k, 13) / 13;
   if ((double)o0 * o1 * nplanes < line) return false;
   const double size = (double)SM_W * ((o0 + SM_W - 1) / SM_W) * o1 * nplanes / line;
-  const double speed = (k <= 5 ? 1.5 : k <= 9 ? 1.2 : 1.05) + std::min(0.35, 0.18 * (size - 1));
+  const double speed = k <= 9 ? (k <= 5 ? 1.6 : 1.2) + std::min(0.35, 0.3 * (size - 1))
+                              : 1.1 + std::min(0.4, 0.18 * (size - 1));
   const MarchFill f(k, o0, o1, SM_MAXROWS);
-  return speed * march_eltype(dt_in, 0.92, 0.82) * (0.25 * f.cover + 0.75 * f.columns) * f.tiled >= f.cover * f.marched;
+  return speed * march_eltype(dt_in, 0.9, 0.85) * (0.15 * f.cover + 0.85 * f.columns) * f.tiled >= f.cover * f.marched;
 }
 
 static bool sep_march_takes(int k0, int k1, int dt_in) {

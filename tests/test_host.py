@@ -282,6 +282,7 @@ def test_separable_march_rule():
             assert took == sorted(took)
         assert pays(k, F32, 4096, line // 4096 + 1, 1)
     assert not pays(21, BF16, 4096, 6_500_000 // 4096 + 1, 1)
+    assert pays(29, BF16, 4096, 4096, 1) and pays(33, F16, 4096, 4096, 1)
 
 
 def test_separable_march_rule_of_batches():
