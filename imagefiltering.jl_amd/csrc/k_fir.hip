@@ -395,14 +395,14 @@ static bool sep_march_takes(int k0, int k1, int dt_in) {
 }
 
 static bool march_launch(const Sep2dArgs &s, hipStream_t st) {
-  if (!sep_march_takes(s.k0, s.k1, s.dt_in)) return false;
+  if (!sep_march_takes(s.k0, s.k1, s.dt_in) || !sep_march_pays(s.k0, s.dt_in, s.o0, s.o1, s.nplanes)) return false;
   SepMarchArgs m;
   m.s = s;
   m.strips = (s.o0 + SM_W - 1) / SM_W;
   m.rows = march_rows(s.o1, (int64_t)m.strips * s.nplanes, s.k0);
   m.chunks = (s.o1 + m.rows - 1) / m.rows;
   m.waves = (int64_t)m.strips * m.chunks * s.nplanes;
-  if (!sep_march_pays(s.k0, s.dt_in, s.o0, s.o1, s.nplanes) || m.waves > (int64_t(1) << 31)) return false;
+  if (m.waves > (int64_t(1) << 31)) return false;
   const dim3 grid((unsigned)((m.waves + 3) / 4));
   switch (s.k0) {
 #define MARCH(K) \
